@@ -255,32 +255,35 @@ int Engine::set_boundary(const int *nbnd, float dt_, float vmax_) {
   return KLRTM_OK;
 }
 
-// effective tile: the values set through klrtm_kernel_set_tile, the defaults for the rest
-void Engine::default_tile(int R, long want, int &etz, int &etx, int &eyc, bool first_deriv) const {
-  // Laplacian step: 64 z lanes (one wave per x row) by 8 x rows.  The first-derivative kernels keep two
-  // halo'd tiles per plane and run fastest on 16 x 16 tiles with 32-plane y chunks (measured on
-  // MI355X at 400^3 and 600x600x400: FD8 VTI 2.23 -> 1.91 ms, FD16 VTI 2.99 -> 2.63 ms, FD16 TTI
-  // 6.75 -> 5.70 ms per step against 64 x 8 tiles)
-  const int tz0 = first_deriv ? 16 : 64, tx0 = first_deriv ? 16 : 8;
-  etz = tz > 0 ? tz : std::max(R, std::min(tz0, nz));
-  etx = tx > 0 ? tx : std::max(R, tx0);
+// Effective tile: the values set through klrtm_kernel_set_tile, the defaults for the rest: 64 z lanes (one
+// wave per x row) by 8 x rows, and the y chunk whose blocks load the 256 CUs most evenly.  A launch takes about
+// (blocks on the fullest CU + 1) * (planes of a block + 3R): a block's start costs R halo planes on each side and
+// the latency of its first loads, and the last block of a CU runs alone.  At least two blocks a CU where the
+// grid has them.  Sweeps of the chunk (MI355X): TTI FD16 300^3 75 planes (0.79 ms a step; 150 planes 0.93, 32
+// planes 0.91), TTI FD16 600x600x400 150 (3.67; 300: 3.91, 60: 3.93), ISO FD8 400^3 67-100 (0.383; 200: 0.441),
+// ISO FD8 128^3 8 (19.6 us; 16: 22.1, 22: 27), VTI FD8 50x55x60 1-2 (20 us; 32 planes 88 us).
+void Engine::default_tile(int R, int &etz, int &etx, int &eyc) const {
+  etz = tz > 0 ? tz : std::max(R, std::min(64, nz));
+  etx = tx > 0 ? tx : std::max(R, 8);
   while(etz * etx > 512) etx = std::max(R, etx / 2);  // the stencil kernels are built for <= 512 threads
   eyc = ychunk;
-  if(eyc <= 0 && first_deriv) eyc = std::min(ny, std::max(2 * R, 32));
-  if(eyc <= 0) {
-    long tiles = (long)div_up(nz, etz) * div_up(nx, etx);
-    int chunks = (int)std::max(1L, std::min((long)ny, (long)div_up(want, std::max(1L, tiles))));
-    eyc = std::max(std::min(ny, 2 * R), div_up(ny, chunks));
+  if(eyc > 0) return;
+  const long tiles = (long)div_up(nz, etz) * div_up(nx, etx);
+  const bool two = tiles * ny >= 512;
+  long best = 0;
+  for(int n = 1; n <= ny; n++) {
+    const int chunk = div_up(ny, n);
+    const long blocks = tiles * div_up(ny, chunk);
+    if(two && blocks < 512) continue;
+    const long cost = (div_up(blocks, 256) + 1L) * (chunk + 3 * R);
+    if(eyc <= 0 || cost < best) best = cost, eyc = chunk;
   }
 }
 
 void Engine::fill_args(IsoArgs &a, int deriv_order) {
   memset(&a, 0, sizeof(a));
   a.nx = nx, a.ny = ny, a.nz = nz;
-  // blocks per launch: the Laplacian step keeps about three rounds of resident blocks (2 per CU on
-  // 256 CUs), so the tail round is short and chunks stay long (fewer y halo planes re-read); the
-  // first-derivative kernels run best with smaller chunks
-  default_tile(ne, deriv_order == 2 ? 1536 : 2048, a.tz, a.tx, a.ychunk, deriv_order == 1);
+  default_tile(ne, a.tz, a.tx, a.ychunk);
   a.do_y = ny > 2;
   a.has_pml = has_pml;
   a.pml = desc;
@@ -484,7 +487,7 @@ int klrtm_kernel_get_tile(klrtm_kernel *kk, int *tz, int *tx, int *ychunk) {
   Engine *k = reinterpret_cast<Engine *>(kk);
   KL_REQUIRE(k, KLRTM_EINVAL, "null engine");
   int a, b, c;
-  k->default_tile(k->ne, 1536, a, b, c);  // as the Laplacian step would run
+  k->default_tile(k->ne, a, b, c);
   if(tz) *tz = a;
   if(tx) *tx = b;
   if(ychunk) *ychunk = c;

@@ -11,58 +11,14 @@
 // iso_step: KernelCPU::ISO Laplacian branch + PML (bgprtm/KernelCPU.cpp:125-174,
 //           bgprtm/FdEngine_fd.cpp:204-325, bgprtm/FdEngine.cpp:352-395) with
 //           Propagator::update2nd fused (bgprtm/Propagator.cpp:1767-1788).
-// grad:     first-derivative gradient + PML round 1 + ScalarVTI/ScalarTTI
-//           (bgprtm/KernelCPU.cpp:93-119,176-297, bgprtm/FdEngine_fd.cpp:388-470).
-// div:      divergence + PML round 2 + pb -= vel*div (+ update2nd).
+// The first-derivative form (VTI, TTI, density) is in fd_grad_kernels.hip and fd_div_kernels.hip.
 #include "klrtm_internal.h"
 #include "fd_kernels.h"
+#include "fd_tile.h"
 #include "stencil_common.h"
 #include <type_traits>
 
 namespace klrtm {
-
-// ---------------------------------------------------------------------------
-// Common tile bookkeeping and the one-plane-ahead prefetch of a cross-shaped
-// halo (z halo of the own row, x halo of the own column).
-struct TileCoord {
-  int tz, tx, iz, ix, y0, y1;
-  bool act;
-  size_t col;
-};
-__device__ __forceinline__ TileCoord tile_coord(const IsoArgs &a) {
-  TileCoord c;
-  // Consecutive logical tiles run together on one XCD (xcd_remap); z tiles vary fastest, so the
-  // co-resident set is a patch of whole z columns over neighbouring x: the z and x halos a block
-  // reads are mostly its neighbours' rows, already in that XCD's L2.
-  int t = xcd_remap(blockIdx.x, gridDim.x);
-  const int bz = t % a.nbz;
-  t /= a.nbz;
-  const int bx = t % a.nbx;
-  const int by = t / a.nbx;
-  c.tz = threadIdx.x % a.tz, c.tx = threadIdx.x / a.tz;
-  c.iz = bz * a.tz + c.tz, c.ix = bx * a.tx + c.tx;
-  c.y0 = by * a.ychunk, c.y1 = min(a.ny, c.y0 + a.ychunk);
-  c.act = c.iz < a.nz && c.ix < a.nx;
-  c.col = (size_t)c.ix * a.nz + c.iz;
-  return c;
-}
-struct Halo {
-  float z0, z1, x0, x1;
-};
-template<int R>
-__device__ __forceinline__ Halo load_halo(const float *__restrict__ u, size_t pl, const TileCoord &c, const IsoArgs &a,
-                                          bool zh, bool xh) {
-  Halo h = {0.f, 0.f, 0.f, 0.f};
-  if(zh) {
-    if(c.tz < R && c.ix < a.nx && c.iz - R >= 0) h.z0 = u[pl + c.col - R];
-    if(c.tz >= a.tz - R && c.ix < a.nx && c.iz + R < a.nz) h.z1 = u[pl + c.col + R];
-  }
-  if(xh) {
-    if(c.tx < R && c.iz < a.nz && c.ix - R >= 0) h.x0 = u[pl + c.col - (size_t)R * a.nz];
-    if(c.tx >= a.tx - R && c.iz < a.nz && c.ix + R < a.nx) h.x1 = u[pl + c.col + (size_t)R * a.nz];
-  }
-  return h;
-}
 
 // ---------------------------------------------------------------------------
 // ISO Laplacian step, streaming version.
@@ -187,20 +143,20 @@ __global__ void __launch_bounds__(512) iso_step_kernel(const float *__restrict__
       const __amdgpu_buffer_rsrc_t ru = prs(u, y);
       N.qa = buf_ld(prs(u, min(y + R, ny - 1)), y + R < ny ? oc : OOR, 0);
       if(MODE != MODE_LAP) {
-        N.w = buf_ld_nt(prs(w0, y), oc, 0);
-        N.v = buf_ld_nt(prs(vel, y), oc, 0);
+        N.w = buf_ld(prs(w0, y), oc, 0);
+        N.v = buf_ld(prs(vel, y), oc, 0);
       }
       N.hz0 = buf_ld(ru, oz0, 0), N.hz1 = buf_ld(ru, oz1, 0);
       N.hx0 = buf_ld(ru, ox0, 0), N.hx1 = buf_ld(ru, ox1, 0);
 #pragma unroll
       for(int r = 0; r < 2; r++) {
-        if(ZL) N.sz[r] = buf_ld_nt(rq[0][r], zo == OOR ? OOR : zo + (uint32_t)y * zs, 0);
-        if(XL) N.sx[r] = buf_ld_nt(rq[1][r], xo == OOR ? OOR : xo + (uint32_t)y * xs, 0);
+        if(ZL) N.sz[r] = buf_ld(rq[0][r], zo == OOR ? OOR : zo + (uint32_t)y * zs, 0);
+        if(XL) N.sx[r] = buf_ld(rq[1][r], xo == OOR ? OOR : xo + (uint32_t)y * xs, 0);
       }
       if(YL) {
         const uint32_t so = (yoff + (uint32_t)(y - jy0) * (uint32_t)nxz) * 4u;
 #pragma unroll
-        for(int r = 0; r < 2; r++) N.sy[r] = buf_ld_nt(rq[2][r], oc, so);
+        for(int r = 0; r < 2; r++) N.sy[r] = buf_ld(rq[2][r], oc, so);
       }
     };
     // plane y: the loads of y+2 go out first; y's tile goes to LDS buffer y&1 (the barrier of y-1
@@ -254,31 +210,31 @@ __global__ void __launch_bounds__(512) iso_step_kernel(const float *__restrict__
         float Lz = round2(zc[0], zc[1], zc[2], L, s1, s2);
         L = zo != OOR ? Lz : L;
         const uint32_t o = zo == OOR ? OOR : zo + (uint32_t)y * zs;
-        buf_st_nt(s1, rq[0][0], o, 0), buf_st_nt(s2, rq[0][1], o, 0);
+        buf_st(s1, rq[0][0], o, 0), buf_st(s2, rq[0][1], o, 0);
       }
       if(XL) {
         float s1 = C.sx[0], s2 = C.sx[1];
         float Lx = round2(xc[0], xc[1], xc[2], L, s1, s2);
         L = xo != OOR ? Lx : L;
         const uint32_t ox = xo == OOR ? OOR : xo + (uint32_t)y * xs;
-        buf_st_nt(s1, rq[1][0], ox, 0), buf_st_nt(s2, rq[1][1], ox, 0);
+        buf_st(s1, rq[1][0], ox, 0), buf_st(s2, rq[1][1], ox, 0);
       }
       if(YL) {
         const cfloat *t = (const cfloat *)P.abc[fy][0] + 3 * (y - jy0);
         float s1 = C.sy[0], s2 = C.sy[1];
         L = round2(t[0], t[1], t[2], L, s1, s2);
         const uint32_t so = (yoff + (uint32_t)(y - jy0) * (uint32_t)nxz) * 4u;
-        buf_st_nt(s1, rq[2][0], oc, so), buf_st_nt(s2, rq[2][1], oc, so);
+        buf_st(s1, rq[2][0], oc, so), buf_st(s2, rq[2][1], oc, so);
       }
       if(MODE == MODE_STEP) {
-        buf_st_nt((ctr + ctr) - fmaf(-C.v, L, C.w), prs(w0, y), oc, 0);
+        buf_st((ctr + ctr) - fmaf(-C.v, L, C.w), prs(w0, y), oc, 0);
       } else if(MODE == MODE_KERNEL) {
-        buf_st_nt(L, prs(pr, y), oc, 0);
-        buf_st_nt(fmaf(-L, C.v, C.w), prs(w0, y), oc, 0);
+        buf_st(L, prs(pr, y), oc, 0);
+        buf_st(fmaf(-L, C.v, C.w), prs(w0, y), oc, 0);
       } else if(MODE == MODE_PB) {
-        buf_st_nt(fmaf(-L, C.v, C.w), prs(w0, y), oc, 0);
+        buf_st(fmaf(-L, C.v, C.w), prs(w0, y), oc, 0);
       } else {
-        buf_st_nt(L, prs(pr, y), oc, 0);
+        buf_st(L, prs(pr, y), oc, 0);
       }
 #pragma unroll
       for(int k = 0; k < 2 * R; k++) q[k] = q[k + 1];
@@ -310,236 +266,6 @@ __global__ void __launch_bounds__(512) iso_step_kernel(const float *__restrict__
   if(c.y0 < s1e) run(T_(), c.y0, s1e, FY1, 0);
   if(s1e < s3b) run(F_(), s1e, s3b, 0, 0);
   if(s3b < c.y1) run(T_(), s3b, c.y1, FY2, ny - wy2);
-}
-
-// ---------------------------------------------------------------------------
-// Gradient + PML round 1 + scalar operator.  Writes px, py (= pr), pz.
-template<int R, int MODEL, bool RHO>
-__global__ void __launch_bounds__(512) grad_kernel(const float *__restrict__ u, float *__restrict__ px,
-                                                    float *__restrict__ py, float *__restrict__ pz,
-                                                    const float *__restrict__ eps, const float *__restrict__ del,
-                                                    const float *__restrict__ pjx, const float *__restrict__ pjy,
-                                                    const IsoArgs a) {
-  extern __shared__ float s[];
-  const int S = a.tz + 2 * R;
-  const int nx = a.nx, ny = a.ny, nz = a.nz;
-  const size_t nxz = (size_t)nx * nz;
-  const TileCoord c = tile_coord(a);
-  const int ix = c.ix, iz = c.iz;
-  const bool do_y = ny > 1;
-  float q[2 * R + 1];
-#pragma unroll
-  for(int k = 0; k < 2 * R; k++) {
-    int yy = c.y0 - R + k;
-    q[k] = (c.act && yy >= 0 && yy < ny) ? u[(size_t)yy * nxz + c.col] : 0.f;
-  }
-  float *srow = s + (c.tx + R) * S + c.tz + R;
-  // irregular z grid: this block's per-iz first-derivative weights, after the tile
-  const bool irr = a.zc1 != nullptr;
-  float *zct = s + (size_t)(a.tx + 2 * R) * S + c.tz * (R + 1);
-  if(irr) {
-    if(c.tx == 0) {
-      const float *g = a.zc1 + (size_t)min(iz, nz - 1) * ZC1_STRIDE;
-#pragma unroll
-      for(int m = 1; m <= R; m++) zct[m] = g[m];
-    }
-    lds_barrier();
-  }
-  float qn = 0.f;
-  Halo hn = load_halo<R>(u, (size_t)c.y0 * nxz, c, a, true, true);
-  if(c.act && c.y0 + R < ny) qn = u[(size_t)(c.y0 + R) * nxz + c.col];
-  // the model parameters of a plane are loaded one plane ahead, with its halos
-  float en = 0.f, dn = 0.f, axn = 0.f, ayn = 0.f;
-  auto model_ld = [&](size_t p) {
-    if(c.act && MODEL != KLRTM_ISO) en = eps[p + c.col], dn = del[p + c.col];
-    if(c.act && MODEL == KLRTM_TTI) axn = pjx[p + c.col], ayn = do_y ? pjy[p + c.col] : 0.f;
-  };
-  model_ld((size_t)c.y0 * nxz);
-  for(int iy = c.y0; iy < c.y1; iy++) {
-    const size_t pl = (size_t)iy * nxz;
-    q[2 * R] = qn;
-    const Halo h = hn;
-    const float e = en, d = dn, ax = axn, ay = ayn;
-    if(iy + 1 < c.y1) {
-      const size_t pn = pl + nxz;
-      hn = load_halo<R>(u, pn, c, a, true, true);
-      if(c.act) qn = (iy + 1 + R < ny) ? u[pn + (size_t)R * nxz + c.col] : 0.f;
-      model_ld(pn);
-    }
-    lds_barrier();
-    srow[0] = q[R];
-    if(c.tz < R) srow[-R] = h.z0;
-    if(c.tz >= a.tz - R) srow[R] = h.z1;
-    if(c.tx < R) srow[-R * S] = h.x0;
-    if(c.tx >= a.tx - R) srow[R * S] = h.x1;
-    lds_barrier();
-    if(c.act) {
-      // z: vz accumulates (-c_m) u[-m] for m=R..1, then c_m u[+m] (bgprtm/FdEngine_fd.cpp:394-403)
-      float gz = 0.f;
-      if(irr) {
-#pragma unroll
-        for(int m = R; m >= 1; m--) gz = fmaf(-zct[m], srow[-m], gz);
-#pragma unroll
-        for(int m = 1; m <= R; m++) gz = fmaf(zct[m], srow[m], gz);
-      } else {
-#pragma unroll
-        for(int m = R; m >= 1; m--) gz = fmaf(-a.cz[m], srow[-m], gz);
-#pragma unroll
-        for(int m = 1; m <= R; m++) gz = fmaf(a.cz[m], srow[m], gz);
-      }
-      // x: vx -= c u[-m]; vx += c u[+m] (bgprtm/FdEngine_fd.cpp:420-431)
-      float gx = 0.f;
-#pragma unroll
-      for(int m = 1; m <= R; m++) {
-        gx = fmaf(-a.cx[m], srow[-m * S], gx);
-        gx = fmaf(a.cx[m], srow[m * S], gx);
-      }
-      float gy = 0.f;
-      if(do_y) {
-#pragma unroll
-        for(int m = 1; m <= R; m++) {
-          gy = fmaf(-a.cy[m], q[R - m], gy);
-          gy = fmaf(a.cy[m], q[R + m], gy);
-        }
-      }
-      if(a.has_pml) {
-        gz = pml1_z<true>(a.pml, 0, gz, ix, iy, iz, nx, ny, nz);
-        gx = pml1_x<true>(a.pml, 0, gx, ix, iy, iz, nx, ny, nz);
-        if(do_y) gy = pml1_y<true>(a.pml, 0, gy, ix, iy, iz, nx, ny, nz);
-      }
-      const size_t i = pl + c.col;
-      if(RHO) {  // KernelCPU::divideRho before the scalar operator (bgprtm/KernelCPU.cpp:103, 340-349)
-        const float r = a.rho[i];
-        gx /= r;
-        if(do_y) gy /= r;
-        gz /= r;
-      }
-      if(MODEL == KLRTM_VTI) scalar_vti(e, d, gx, gy, gz);
-      else if(MODEL == KLRTM_TTI) scalar_tti(e, d, ax, ay, gx, gy, gz);
-      px[i] = gx;
-      if(do_y) py[i] = gy;
-      pz[i] = gz;
-    }
-#pragma unroll
-    for(int k = 0; k < 2 * R; k++) q[k] = q[k + 1];
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Divergence + PML round 2 + pb -= vel*div (x, z, then y as the reference)
-// (+ update2nd in MODE_STEP).  Dx needs x-neighbours of px, Dz z-neighbours of
-// pz, Dy y-neighbours of py: two LDS tiles and one register queue.
-template<int R, int MODE, bool RHO>
-__global__ void __launch_bounds__(512) div_kernel(const float *__restrict__ px, const float *__restrict__ py,
-                                                   const float *__restrict__ pz, const float *__restrict__ w1,
-                                                   float *__restrict__ w0, const float *__restrict__ vel,
-                                                   const IsoArgs a) {
-  extern __shared__ float s[];
-  const int TZ = a.tz, TX = a.tx;
-  const int SZ = TZ + 2 * R;  // row stride of the z-haloed tile (pz)
-  float *sz = s;                // TX rows x (TZ+2R)
-  float *sx = s + TX * SZ;      // (TX+2R) rows x TZ
-  const int nx = a.nx, ny = a.ny, nz = a.nz;
-  const size_t nxz = (size_t)nx * nz;
-  const TileCoord c = tile_coord(a);
-  const int ix = c.ix, iz = c.iz;
-  const bool do_y = ny > 1;
-  float q[2 * R + 1];
-#pragma unroll
-  for(int k = 0; k < 2 * R; k++) {
-    int yy = c.y0 - R + k;
-    q[k] = (do_y && c.act && yy >= 0 && yy < ny) ? py[(size_t)yy * nxz + c.col] : 0.f;
-  }
-  float *zrow = sz + c.tx * SZ + c.tz + R;
-  float *xrow = sx + (c.tx + R) * TZ + c.tz;
-  // irregular z grid: this block's per-iz first-derivative weights, after the two tiles
-  const bool irr = a.zc1 != nullptr;
-  float *zct = sx + (size_t)(TX + 2 * R) * TZ + c.tz * (R + 1);
-  if(irr) {
-    if(c.tx == 0) {
-      const float *g = a.zc1 + (size_t)min(iz, nz - 1) * ZC1_STRIDE;
-#pragma unroll
-      for(int m = 1; m <= R; m++) zct[m] = g[m];
-    }
-    lds_barrier();
-  }
-  auto fetch = [&](size_t p, float &qv, float &cz, float &cx, Halo &hz, Halo &hx, float &wv, float &vv, float &uv,
-                   float &rv, int iyp) {
-    hz = load_halo<R>(pz, p, c, a, true, false);
-    hx = load_halo<R>(px, p, c, a, false, true);
-    if(c.act) {
-      qv = (do_y && iyp + R < ny) ? py[p + (size_t)R * nxz + c.col] : 0.f;
-      cz = pz[p + c.col], cx = px[p + c.col];
-      wv = w0[p + c.col], vv = vel[p + c.col];
-      if(MODE == MODE_STEP) uv = w1[p + c.col];
-      if(RHO) rv = a.rho[p + c.col];
-    }
-  };
-  float qn = 0.f, czn = 0.f, cxn = 0.f, wn = 0.f, vn = 0.f, un = 0.f, rn = 1.f;
-  Halo hzn, hxn;
-  fetch((size_t)c.y0 * nxz, qn, czn, cxn, hzn, hxn, wn, vn, un, rn, c.y0);
-  for(int iy = c.y0; iy < c.y1; iy++) {
-    const size_t pl = (size_t)iy * nxz;
-    q[2 * R] = qn;
-    const float cz = czn, cx = cxn, wv = wn, vv = vn, uv = un, rv = rn;
-    const Halo hz = hzn, hx = hxn;
-    if(iy + 1 < c.y1) fetch(pl + nxz, qn, czn, cxn, hzn, hxn, wn, vn, un, rn, iy + 1);
-    lds_barrier();
-    zrow[0] = cz;
-    if(c.tz < R) zrow[-R] = hz.z0;
-    if(c.tz >= TZ - R) zrow[R] = hz.z1;
-    xrow[0] = cx;
-    if(c.tx < R) xrow[-R * TZ] = hx.x0;
-    if(c.tx >= TX - R) xrow[R * TZ] = hx.x1;
-    lds_barrier();
-    if(c.act) {
-      float dxv = 0.f;
-#pragma unroll
-      for(int m = 1; m <= R; m++) {
-        dxv = fmaf(-a.cx[m], xrow[-m * TZ], dxv);
-        dxv = fmaf(a.cx[m], xrow[m * TZ], dxv);
-      }
-      float dzv = 0.f;
-      if(irr) {
-#pragma unroll
-        for(int m = R; m >= 1; m--) dzv = fmaf(-zct[m], zrow[-m], dzv);
-#pragma unroll
-        for(int m = 1; m <= R; m++) dzv = fmaf(zct[m], zrow[m], dzv);
-      } else {
-#pragma unroll
-        for(int m = R; m >= 1; m--) dzv = fmaf(-a.cz[m], zrow[-m], dzv);
-#pragma unroll
-        for(int m = 1; m <= R; m++) dzv = fmaf(a.cz[m], zrow[m], dzv);
-      }
-      float dyv = 0.f;
-      if(do_y) {
-#pragma unroll
-        for(int m = 1; m <= R; m++) {
-          dyv = fmaf(-a.cy[m], q[R - m], dyv);
-          dyv = fmaf(a.cy[m], q[R + m], dyv);
-        }
-      }
-      if(a.has_pml) {
-        dxv = pml1_x<true>(a.pml, 1, dxv, ix, iy, iz, nx, ny, nz);
-        dzv = pml1_z<true>(a.pml, 1, dzv, ix, iy, iz, nx, ny, nz);
-        if(do_y) dyv = pml1_y<true>(a.pml, 1, dyv, ix, iy, iz, nx, ny, nz);
-      }
-      float w;
-      if(RHO) {  // out -= d*vel*rho (bgprtm/FdEngine_fd.cpp:409-412, 435-438, 461-464)
-        w = fmaf(-(dxv * vv), rv, wv);
-        w = fmaf(-(dzv * vv), rv, w);
-        if(do_y) w = fmaf(-(dyv * vv), rv, w);
-      } else {
-        w = fmaf(-dxv, vv, wv);
-        w = fmaf(-dzv, vv, w);
-        if(do_y) w = fmaf(-dyv, vv, w);
-      }
-      if(MODE == MODE_STEP) w = (uv + uv) - w;
-      w0[pl + c.col] = w;
-    }
-#pragma unroll
-    for(int k = 0; k < 2 * R; k++) q[k] = q[k + 1];
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -604,12 +330,6 @@ int launch_deriv1(int R, int axis, int iacc, int round, const float *in, float *
 
 // ---------------------------------------------------------------------------
 // host launchers
-static void grid_of(IsoArgs &a) {
-  a.nbz = div_up(a.nz, a.tz);
-  a.nbx = div_up(a.nx, a.tx);
-  a.nby = div_up(a.ny, a.ychunk);
-}
-
 template<int R, int MODE>
 static int launch_iso_rm(const float *u, float *w0, const float *vel, float *pr, const IsoArgs &a, int nb, size_t lds) {
   hipLaunchKernelGGL((iso_step_kernel<R, MODE>), dim3(nb), dim3(a.tz * a.tx), lds, stream(), u, w0, vel, pr, a);
@@ -636,72 +356,6 @@ int launch_iso(int R, int mode, const float *u, float *w0, const float *vel, flo
   case 6: return launch_iso_r<6>(mode, u, w0, vel, pr, a);
   case 7: return launch_iso_r<7>(mode, u, w0, vel, pr, a);
   case 8: return launch_iso_r<8>(mode, u, w0, vel, pr, a);
-  default: set_error("FD half order %d not supported (4..8)", R); return KLRTM_EINVAL;
-  }
-}
-
-template<int R, int MODEL>
-static int launch_grad_rm(const float *u, float *px, float *py, float *pz, const float *eps, const float *del,
-                          const float *pjx, const float *pjy, IsoArgs a) {
-  grid_of(a);
-  int nb = a.nbz * a.nbx * a.nby;
-  size_t lds = sizeof(float) * (size_t)(a.tx + 2 * R) * (a.tz + 2 * R);
-  if(a.zc1) lds += sizeof(float) * (size_t)a.tz * (R + 1);
-  LaunchTimer tm("fd_grad");
-  if(a.rho)
-    hipLaunchKernelGGL((grad_kernel<R, MODEL, true>), dim3(nb), dim3(a.tz * a.tx), lds, stream(), u, px, py, pz, eps, del,
-                       pjx, pjy, a);
-  else
-    hipLaunchKernelGGL((grad_kernel<R, MODEL, false>), dim3(nb), dim3(a.tz * a.tx), lds, stream(), u, px, py, pz, eps, del,
-                       pjx, pjy, a);
-  return check_launch("grad_kernel");
-}
-template<int R>
-static int launch_grad_r(int model, const float *u, float *px, float *py, float *pz, const float *eps,
-                         const float *del, const float *pjx, const float *pjy, const IsoArgs &a) {
-  if(model == KLRTM_VTI) return launch_grad_rm<R, KLRTM_VTI>(u, px, py, pz, eps, del, pjx, pjy, a);
-  if(model == KLRTM_TTI) return launch_grad_rm<R, KLRTM_TTI>(u, px, py, pz, eps, del, pjx, pjy, a);
-  return launch_grad_rm<R, KLRTM_ISO>(u, px, py, pz, eps, del, pjx, pjy, a);
-}
-int launch_grad(int R, int model, const float *u, float *px, float *py, float *pz, const float *eps, const float *del,
-                const float *pjx, const float *pjy, const IsoArgs &a) {
-  switch(R) {
-  case 4: return launch_grad_r<4>(model, u, px, py, pz, eps, del, pjx, pjy, a);
-  case 5: return launch_grad_r<5>(model, u, px, py, pz, eps, del, pjx, pjy, a);
-  case 6: return launch_grad_r<6>(model, u, px, py, pz, eps, del, pjx, pjy, a);
-  case 7: return launch_grad_r<7>(model, u, px, py, pz, eps, del, pjx, pjy, a);
-  case 8: return launch_grad_r<8>(model, u, px, py, pz, eps, del, pjx, pjy, a);
-  default: set_error("FD half order %d not supported (4..8)", R); return KLRTM_EINVAL;
-  }
-}
-
-template<int R>
-static int launch_div_r(int mode, const float *px, const float *py, const float *pz, const float *w1, float *w0,
-                        const float *vel, IsoArgs a) {
-  grid_of(a);
-  int nb = a.nbz * a.nbx * a.nby;
-  size_t lds = sizeof(float) * ((size_t)a.tx * (a.tz + 2 * R) + (size_t)(a.tx + 2 * R) * a.tz);
-  if(a.zc1) lds += sizeof(float) * (size_t)a.tz * (R + 1);
-  LaunchTimer tm(mode == MODE_STEP ? "fd_div_step" : "fd_div");
-  const dim3 g(nb), b(a.tz * a.tx);
-  if(mode == MODE_STEP && a.rho)
-    hipLaunchKernelGGL((div_kernel<R, MODE_STEP, true>), g, b, lds, stream(), px, py, pz, w1, w0, vel, a);
-  else if(mode == MODE_STEP)
-    hipLaunchKernelGGL((div_kernel<R, MODE_STEP, false>), g, b, lds, stream(), px, py, pz, w1, w0, vel, a);
-  else if(a.rho)
-    hipLaunchKernelGGL((div_kernel<R, MODE_KERNEL, true>), g, b, lds, stream(), px, py, pz, w1, w0, vel, a);
-  else
-    hipLaunchKernelGGL((div_kernel<R, MODE_KERNEL, false>), g, b, lds, stream(), px, py, pz, w1, w0, vel, a);
-  return check_launch("div_kernel");
-}
-int launch_div(int R, int mode, const float *px, const float *py, const float *pz, const float *w1, float *w0,
-               const float *vel, const IsoArgs &a) {
-  switch(R) {
-  case 4: return launch_div_r<4>(mode, px, py, pz, w1, w0, vel, a);
-  case 5: return launch_div_r<5>(mode, px, py, pz, w1, w0, vel, a);
-  case 6: return launch_div_r<6>(mode, px, py, pz, w1, w0, vel, a);
-  case 7: return launch_div_r<7>(mode, px, py, pz, w1, w0, vel, a);
-  case 8: return launch_div_r<8>(mode, px, py, pz, w1, w0, vel, a);
   default: set_error("FD half order %d not supported (4..8)", R); return KLRTM_EINVAL;
   }
 }
