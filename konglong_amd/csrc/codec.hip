@@ -23,61 +23,123 @@ __global__ void fill_u32_kernel(unsigned *p, unsigned v, int n) {
   if(i < n) p[i] = v;
 }
 
+// W codes (2W bytes) per thread: the codes of a slice start 4 bytes after its slice header, so a slice's first
+// codes up to a 2W-byte boundary of the code stream form a chunk of their own (chunk 0), and chunk c > 0 is codes
+// lead + W(c-1).. .  The float side is then only 4-byte aligned, which the hardware's wide accesses accept.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+struct C16Chunk {
+  size_t j0;   // first code of the chunk in its slice
+  unsigned n;  // codes in it (0: past the end)
+};
+template<int W> __device__ __forceinline__ C16Chunk c16_chunk(const uint16_t *codes, size_t nxz, size_t c) {
+  const size_t lead = min(nxz, (size_t)(((2 * W - ((uintptr_t)codes & (2 * W - 1))) & (2 * W - 1)) / 2));
+  C16Chunk k;
+  if(c == 0) k.j0 = 0, k.n = (unsigned)lead;
+  else k.j0 = lead + (c - 1) * W, k.n = k.j0 < nxz ? (unsigned)min((size_t)W, nxz - k.j0) : 0u;
+  return k;
+}
+static unsigned c16_blocks(size_t nxz, int W) { return (unsigned)(((nxz + W - 1) / W + 1 + 255) / 256); }
+constexpr int C16_ENC = 8, C16_DEC = 4;  // (a wave's stores are contiguous: 16 bytes a lane on either side)
+constexpr int C16_DEC_U = 4;             // decode chunks per thread
+constexpr int C16_GRID_Y = 65535;  // slices per launch
+
 // per-slice max |x| (bgprtm/WaveFieldCompress.cpp:149-153); non-negative FP32
 // compare like their bit patterns, so atomicMax on the bits is exact and
-// order independent.
-__global__ void slice_absmax_kernel(const float *__restrict__ in, size_t nxz, unsigned *__restrict__ smax) {
+// order independent.  A slice that one workgroup covers is stored without it.
+__global__ void __launch_bounds__(256) slice_absmax_kernel(const float *__restrict__ in, size_t nxz,
+                                                           unsigned *__restrict__ smax) {
   const int iy = blockIdx.y;
   const float *p = in + (size_t)iy * nxz;
+  const size_t n4 = nxz / 4;
   float m = 0.f;
-  for(size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < nxz; i += (size_t)gridDim.x * blockDim.x)
-    m = fmaxf(m, fabsf(p[i]));
+  const size_t step = (size_t)gridDim.x * 256;
+  for(size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += 4 * step) {
+    f4u v[4];  // in flight together; past the end the last quad again
+#pragma unroll
+    for(int u = 0; u < 4; u++) v[u] = *(const f4u *)(p + 4 * min(i + u * step, n4 - 1));
+#pragma unroll
+    for(int u = 0; u < 4; u++)
+      m = fmaxf(fmaxf(m, fmaxf(fabsf(v[u].x), fabsf(v[u].y))), fmaxf(fabsf(v[u].z), fabsf(v[u].w)));
+  }
+  if(blockIdx.x == 0 && threadIdx.x < nxz - 4 * n4) m = fmaxf(m, fabsf(p[4 * n4 + threadIdx.x]));
   for(int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  __shared__ float red[16];
+  __shared__ float red[4];
   int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if(lane == 0) red[wid] = m;
   __syncthreads();
   if(threadIdx.x == 0) {
-    float r = 0.f;
-    for(int w = 0; w < (int)(blockDim.x >> 6); w++) r = fmaxf(r, red[w]);
-    atomicMax(&smax[iy], __float_as_uint(r));
+    const float r = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if(gridDim.x == 1) smax[iy] = __float_as_uint(r);
+    else atomicMax(&smax[iy], __float_as_uint(r));
   }
 }
 
-__global__ void c16_encode_kernel(const float *__restrict__ in, uint16_t *__restrict__ out, const unsigned *__restrict__ smax,
-                                  size_t nxz, int ny) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if(i >= nxz * ny) return;
-  int iy = (int)(i / nxz);
-  size_t j = i - (size_t)iy * nxz;
-  float vmax = __uint_as_float(smax[iy]);
+// Bound by HBM: 4 bytes in, 2 out per sample.  One sample per thread, 64-bit index division and divergent code
+// ranges ran at 1.8 TB/s (400^3: 217 us); eight samples per thread with 16-byte accesses take 66 us (5.9 TB/s).
+__global__ void __launch_bounds__(256) c16_encode_kernel(const float *__restrict__ in, uint16_t *__restrict__ out,
+                                                         const unsigned *__restrict__ smax, size_t nxz) {
+  const int iy = blockIdx.y;
+  const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
   uint16_t *pout = out + (size_t)iy * (nxz + 2);
-  if(vmax > 1e-25f) {
-    float scale = 1.0f / vmax;
-    pout[2 + j] = c16_shift(in[i] * scale);
-    if(j == 0) {
-      unsigned b = __float_as_uint(vmax);
-      pout[0] = (uint16_t)(b & 0xffffu), pout[1] = (uint16_t)(b >> 16);
-    }
+  const C16Chunk k = c16_chunk<C16_ENC>(pout + 2, nxz, c);
+  const float vmax = __uint_as_float(smax[iy]);
+  const bool on = vmax > 1e-25f;
+  if(c == 0) {
+    const unsigned b = on ? __float_as_uint(vmax) : 0u;
+    pout[0] = (uint16_t)(b & 0xffffu), pout[1] = (uint16_t)(b >> 16);
+  }
+  const float scale = on ? 1.0f / vmax : 0.f;
+  const float *pin = in + (size_t)iy * nxz + k.j0;
+  if(k.n == C16_ENC) {
+    const f4u a = *(const f4u *)pin, b = *(const f4u *)(pin + 4);
+    auto two = [&](float x, float y) {
+      const unsigned u = (unsigned)c16_shift(x * scale) | (unsigned)c16_shift(y * scale) << 16;
+      return on ? u : 0u;
+    };
+    *(uint4 *)(pout + 2 + k.j0) = make_uint4(two(a.x, a.y), two(a.z, a.w), two(b.x, b.y), two(b.z, b.w));
   } else {
-    pout[2 + j] = 0;
-    if(j == 0) pout[0] = 0, pout[1] = 0;
+    for(unsigned j = 0; j < k.n; j++) pout[2 + k.j0 + j] = on ? c16_shift(pin[j] * scale) : (uint16_t)0;
   }
 }
 
-__global__ void c16_decode_kernel(const uint16_t *__restrict__ in, float *__restrict__ out, int nx, int ny, int nz,
-                                  const EdgeTaper T) {
-  size_t nxz = (size_t)nx * nz;
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if(i >= nxz * ny) return;
-  int iy = (int)(i / nxz);
-  size_t j = i - (size_t)iy * nxz;
-  int ix = (int)(j / nz), iz = (int)(j - (size_t)ix * nz);
+// 2 bytes in, 4 out per sample.  The edge taper's factors (one per axis; the low and high edges do not overlap) come
+// from a table in LDS that holds 1 past the taper: nearly every wave reaches a tapered z, and reading the factors
+// from the arguments under a branch cost more than the volume (400^3: 277 us, now about 85).
+__global__ void __launch_bounds__(256) c16_decode_kernel(const uint16_t *__restrict__ in, float *__restrict__ out, int nx,
+                                                         int ny, int nz, int y0, const EdgeTaper T) {
+  __shared__ float wt[21], wzt[11];
+  if(threadIdx.x < 20) wt[threadIdx.x] = T.wt[threadIdx.x];
+  if(threadIdx.x < 10) wzt[threadIdx.x] = T.wzt[threadIdx.x];
+  if(threadIdx.x == 0) wt[20] = wzt[10] = 1.f;
+  __syncthreads();
+  const size_t nxz = (size_t)nx * nz;
+  const int iy = y0 + (int)blockIdx.y;
   const uint16_t *pin = in + (size_t)iy * (nxz + 2);
-  float scale = __uint_as_float((unsigned)pin[0] | ((unsigned)pin[1] << 16));
-  float v = 0.f;
-  if(scale > 1e-25f) v = edge_taper(T, scale * c16_value(pin[2 + j]), ix, iy, iz, nx, ny, nz);
-  out[i] = v;
+  const float scale = __uint_as_float((unsigned)pin[0] | ((unsigned)pin[1] << 16));
+  const bool on = scale > 1e-25f;
+  const float fy = ny > 40 ? wt[min(min(iy, ny - 1 - iy), 20)] : 1.f;
+#pragma unroll
+  for(int u = 0; u < C16_DEC_U; u++) {
+    const C16Chunk k = c16_chunk<C16_DEC>(pin + 2, nxz, ((size_t)blockIdx.x * C16_DEC_U + u) * 256 + threadIdx.x);
+    if(k.n == 0) continue;  // past the end, or an empty first chunk
+    float *pout = out + (size_t)iy * nxz + k.j0;
+    int ix = nxz >> 32 ? (int)(k.j0 / nz) : (int)((unsigned)k.j0 / (unsigned)nz), iz = (int)(k.j0 - (size_t)ix * nz);
+    auto value = [&](unsigned code) {
+      const float fx = nx > 40 ? wt[min(min(ix, nx - 1 - ix), 20)] : 1.f;
+      const float fz = nz > 20 ? wzt[min(min(iz, nz - 1 - iz), 10)] : 1.f;
+      const float v = scale * c16_value((uint16_t)code);
+      if(++iz == nz) iz = 0, ix++;
+      return on ? v * fy * fx * fz : 0.f;
+    };
+    if(k.n == C16_DEC) {
+      const uint2 q = *(const uint2 *)(pin + 2 + k.j0);
+      f4u v;
+      v.x = value(q.x & 0xffffu), v.y = value(q.x >> 16), v.z = value(q.y & 0xffffu), v.w = value(q.y >> 16);
+      *(f4u *)pout = v;
+    } else {
+      for(unsigned j = 0; j < k.n; j++) pout[j] = value(pin[2 + k.j0 + j]);
+    }
+  }
 }
 
 EdgeTaper make_edge_taper() {
@@ -89,28 +151,36 @@ EdgeTaper make_edge_taper() {
 }
 
 int c16_slice_max(const float *in, int nx, int ny, int nz, unsigned *smax) {
-  size_t nxz = (size_t)nx * nz;
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(div_up(ny, 256)), dim3(256), 0, stream(), smax, 0u, ny);
-  int bx = (int)std::min<size_t>(64, (nxz + 4095) / 4096);
-  hipLaunchKernelGGL(slice_absmax_kernel, dim3(bx, ny), dim3(256), 0, stream(), in, nxz, smax);
+  const size_t nxz = (size_t)nx * nz;
+  // 16 Ki samples a workgroup; a slice of one workgroup needs no cleared maximum
+  const int bx = (int)std::min<size_t>(64, (nxz + 16383) / 16384);
+  if(bx > 1) hipLaunchKernelGGL(fill_u32_kernel, dim3(div_up(ny, 256)), dim3(256), 0, stream(), smax, 0u, ny);
+  for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y)
+    hipLaunchKernelGGL(slice_absmax_kernel, dim3(bx, std::min(ny - y0, C16_GRID_Y)), dim3(256), 0, stream(),
+                       in + (size_t)y0 * nxz, nxz, smax + y0);
   return check_launch("slice_absmax_kernel");
+}
+
+static int c16_encode_slices(const float *in, uint16_t *out, int nx, int ny, int nz, const unsigned *smax) {
+  const size_t nxz = (size_t)nx * nz;
+  for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y)
+    hipLaunchKernelGGL(c16_encode_kernel, dim3(c16_blocks(nxz, C16_ENC), std::min(ny - y0, C16_GRID_Y)), dim3(256), 0, stream(),
+                       in + (size_t)y0 * nxz, out + (size_t)y0 * (nxz + 2), smax + y0, nxz);
+  return check_launch("c16_encode_kernel");
 }
 
 int c16_encode(const float *in, uint16_t *out, int nx, int ny, int nz, unsigned *smax) {
   int rc = c16_slice_max(in, nx, ny, nz, smax);
   if(rc) return rc;
-  size_t n = (size_t)nx * ny * nz;
   LaunchTimer tm("c16_encode");
-  hipLaunchKernelGGL(c16_encode_kernel, dim3((unsigned)div_up((long)n, 256)), dim3(256), 0, stream(), in, out, smax,
-                     (size_t)nx * nz, ny);
-  return check_launch("c16_encode_kernel");
+  return c16_encode_slices(in, out, nx, ny, nz, smax);
 }
 
 int c16_decode(const uint16_t *in, float *out, int nx, int ny, int nz) {
-  size_t n = (size_t)nx * ny * nz;
   LaunchTimer tm("c16_decode");
-  hipLaunchKernelGGL(c16_decode_kernel, dim3((unsigned)div_up((long)n, 256)), dim3(256), 0, stream(), in, out, nx, ny, nz,
-                     make_edge_taper());
+  for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y)
+    hipLaunchKernelGGL(c16_decode_kernel, dim3(div_up(c16_blocks((size_t)nx * nz, C16_DEC), C16_DEC_U), std::min(ny - y0, C16_GRID_Y)), dim3(256), 0,
+                       stream(), in, out, nx, ny, nz, y0, make_edge_taper());
   return check_launch("c16_decode_kernel");
 }
 
@@ -370,10 +440,7 @@ int klrtm_compress16_noalloc(const float *in, uint16_t *out, int nx, int ny, int
   // no launch timer here: it would create events on first use
   rc = c16_slice_max(in, nx, ny, nz, smax);
   if(rc) return rc;
-  const size_t n = (size_t)nx * ny * nz;
-  hipLaunchKernelGGL(c16_encode_kernel, dim3((unsigned)div_up((long)n, 256)), dim3(256), 0, stream(), in, out, smax,
-                     (size_t)nx * nz, ny);
-  return check_launch("c16_encode_kernel");
+  return c16_encode_slices(in, out, nx, ny, nz, smax);
 }
 int klrtm_uncompress16(const uint16_t *in, float *out, int nx, int ny, int nz) {
   KL_REQUIRE(in && out, KLRTM_EINVAL, "null pointer");

@@ -13,44 +13,31 @@
 
 namespace klrtm {
 
+// The three exponent ranges and the special cases as selects: the branches of the reference's form diverge in
+// almost every wave of a wavefield.
 // bgprtm/WaveFieldCompress.cpp:107-133
 __device__ __forceinline__ uint16_t c16_shift(float w) {
-  int idat = __float_as_int(w);
-  uint16_t sgn = (uint16_t)(((unsigned)idat & 0x80000000u) >> 16);
-  int exp = (int)(((unsigned)idat & 0x7f800000u) >> 23) - 127;
-  int frc;
-  if(exp > 0) return 0x8000;
-  if(exp == 0) return sgn | 0x1;
-  if(exp > -5) {
-    frc = (idat & 0x7fffff) | 0x800000;
-    return (uint16_t)(sgn | (frc >> (9 - exp)));
-  }
-  if(exp > -21) {
-    exp += 20;
-    frc = (idat & 0x7fffff);
-    return (uint16_t)(sgn | 0x4000 | (exp << 10) | (frc >> 13));
-  }
-  if(exp > -30) {
-    frc = (idat & 0x7fffff) | 0x800000;
-    return (uint16_t)(sgn | (frc >> (-7 - exp)));
-  }
-  return 0;
+  const unsigned bits = __float_as_uint(w), sgn = (bits >> 16) & 0x8000u, f = bits & 0x7fffffu, g = f | 0x800000u;
+  const int e = (int)((bits >> 23) & 0xffu) - 127;
+  // -4..-1: 2^-14 steps; -20..-5: 10-bit fraction per octave; -29..-21: 2^-30 steps
+  const unsigned lin = sgn | (g >> ((e > -5 ? 9 - e : -7 - e) & 31));
+  const unsigned oct = sgn | 0x4000u | ((unsigned)(e + 20) << 10) | (f >> 13);
+  unsigned r = e > -5 || e < -20 ? lin : oct;
+  r = e < -29 ? 0u : r;
+  r = e == 0 ? (sgn | 1u) : r;
+  return (uint16_t)(e > 0 ? 0x8000u : r);
 }
 
 // value of table[c] (bgprtm/WaveFieldCompress.cpp:52-86)
 __device__ __forceinline__ float c16_value(uint16_t c) {
-  if(c == 0x8000) return __int_as_float(0x7fffffff);
-  unsigned m = c & 0x7fffu;
-  float v;
-  if(m == 0) v = 0.f;
-  else if(m == 1) v = 1.f;
-  else if(m < 1024) v = 0x1p-30f * (float)m;
-  else if(m < 16384) v = 0x1p-14f * (float)m;
-  else {
-    int j = (int)((m - 16384u) >> 10), i = (int)(m & 1023u);
-    v = __int_as_float((127 - (20 - j)) << 23) * (1.f + (float)i * (1.f / 1024.f));
-  }
-  return (c & 0x8000) ? -v : v;
+  const unsigned m = c & 0x7fffu;
+  const float lin = (float)m * (m < 1024u ? 0x1p-30f : 0x1p-14f);
+  // 2^(j-20) * (1 + i/1024), j = (m - 16384) >> 10, i = m & 1023: exact in the float's own fields
+  const float oct = __uint_as_float((((m - 16384u) >> 10) + 107u) << 23 | (m & 1023u) << 13);
+  float v = m < 16384u ? lin : oct;
+  v = m == 1u ? 1.f : v;
+  v = (c & 0x8000u) ? -v : v;
+  return c == 0x8000u ? __uint_as_float(0x7fffffffu) : v;
 }
 
 // edge taper of the decoded wavefield, multiplied in the reference's order:
