@@ -162,17 +162,22 @@ struct GroupArgs {
 // wy[j][k] = (val_r*scaler)*ky_r[j] for the receiver r at CSR position k of
 // the group's nr: the y factor of every term, formed once per step.
 // The trace sample is t = step_index(ts) of traces [nt][nrt]; outside [0, nt) the factors are zero, so
-// the plane is zero and the apply kernels leave the wavefield untouched (as a skipped injection does).
+// the plane is zero and the wavefield is left untouched (as by a skipped injection).
+struct TraceArgs {
+  const float *traces;
+  int nrt, nt;
+  StepRef ts;
+  float scaler;
+};
 __global__ void inject_wy_kernel(int n, int nr, const int *__restrict__ bin_rcv, const float *__restrict__ cky,
-                                 const float *__restrict__ traces, int nrt, int nt, const StepRef ts, float scaler,
-                                 float *__restrict__ wy) {
+                                 const TraceArgs tr, float *__restrict__ wy) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if(e >= n) return;
-  const int t = step_index(ts);
-  wy[e] = t >= 0 && t < nt ? (traces[(size_t)t * nrt + bin_rcv[e % nr]] * scaler) * cky[e] : 0.f;
+  const int t = step_index(tr.ts);
+  wy[e] = t >= 0 && t < tr.nt ? (tr.traces[(size_t)t * tr.nrt + bin_rcv[e % nr]] * tr.scaler) * cky[e] : 0.f;
 }
 
-// T[iy][ix] = sum_r (val_r*ky_r)*kx_r over receivers covering (ix,iy).
+// T of cell c = sum_r (val_r*ky_r)*kx_r over receivers covering it.
 // A receiver can reach a cell only if its kernel origin lies in [cell - lmax
 // + 1, cell] on both axes; for each origin row those receivers are one
 // contiguous CSR range of the bins.  IG adjacent lanes share a cell, lane j
@@ -183,28 +188,33 @@ __global__ void inject_wy_kernel(int n, int nr, const int *__restrict__ bin_rcv,
 // neighbouring receivers at the same tap offsets, so the loads of a wave are
 // contiguous, and there is no bounds branch: an index outside [0, L) is
 // clamped and its term dropped by a select (adding +0 leaves a sum that
-// started at +0 unchanged).
-template<int IG>
-__global__ void __launch_bounds__(256)
-    inject_plane_kernel(const GroupArgs a, const int *__restrict__ bin_start, const int2 *__restrict__ corg,
-                        const float *__restrict__ ckx, const float *__restrict__ wy, float *__restrict__ plane) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int c = (int)(t / IG), sub = (int)(t % IG);
-  const bool act = c < a.bw * a.bh;
-  const int L = a.L;
+// started at +0 unchanged).  The y factor comes from wy, or (WY null) is formed here.
+constexpr int IG = 4;
+struct GatherTabs {
+  const int *bin_start, *bin_rcv;
+  const int2 *corg;
+  const float *ckx, *cky, *wy;
+};
+template<bool WY>
+__device__ __forceinline__ float gather_cell(const GroupArgs &a, const GatherTabs &g, const TraceArgs &tr, int c, int sub) {
   float T = 0.f;
-  if(act) {
+  if(c < a.bw * a.bh) {
+    const int L = a.L, t = WY ? 0 : step_index(tr.ts);
+    const bool on = WY || (t >= 0 && t < tr.nt);
+    const float *row = tr.traces + (size_t)(on ? t : 0) * tr.nrt;
     const int px = c % a.bw, py = c / a.bw;
     const int jx = a.bx0 + px, jy = a.by0 + py;  // absolute cell
     const int qx_lo = max(0, px - a.lxmax + 1), qy_lo = max(0, py - a.lymax + 1);
     for(int qy = qy_lo + sub; qy <= py; qy += IG) {
-      const int k0 = bin_start[qy * a.bw + qx_lo], k1 = bin_start[qy * a.bw + px + 1];
+      const int k0 = g.bin_start[qy * a.bw + qx_lo], k1 = g.bin_start[qy * a.bw + px + 1];
 #pragma unroll 4
       for(int k = k0; k < k1; k++) {
-        const int2 o = corg[k];
+        const int2 o = g.corg[k];
         const int ex = jx - o.x, ey = jy - o.y;
         const bool ok = ex >= 0 && ey >= 0 && ex < L && ey < L;
-        const float term = wy[(size_t)min(max(ey, 0), L - 1) * a.nr + k] * ckx[(size_t)min(max(ex, 0), L - 1) * a.nr + k];
+        const size_t iy = (size_t)min(max(ey, 0), L - 1) * a.nr + k, ix = (size_t)min(max(ex, 0), L - 1) * a.nr + k;
+        const float y = WY ? g.wy[iy] : on ? (row[g.bin_rcv[k]] * tr.scaler) * g.cky[iy] : 0.f;
+        const float term = y * g.ckx[ix];
         T += ok ? term : 0.f;
       }
     }
@@ -212,93 +222,156 @@ __global__ void __launch_bounds__(256)
   // lanes c*IG .. c*IG+IG-1 are adjacent in one wave: (T0 + T1) + (T2 + T3) in every lane
 #pragma unroll
   for(int m = 1; m < IG; m *= 2) T = T + __shfl_xor(T, m);
-  if(act && sub == 0) plane[c] = T;
+  return T;
 }
-constexpr int IG = 4;
+__global__ void __launch_bounds__(256)
+    inject_plane_kernel(const GroupArgs a, const GatherTabs g, const TraceArgs tr, float *__restrict__ plane) {
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  const int c = (int)(t / IG), sub = (int)(t % IG);
+  const float T = gather_cell<true>(a, g, tr, c, sub);
+  if(c < a.bw * a.bh && sub == 0) plane[c] = T;
+}
 
-// Separable form of the same plane.  v[k] = val*scaler of row receiver k (zero outside the record).
-__global__ void inject_val_kernel(int n, const int *__restrict__ rrid, const float *__restrict__ traces, int nrt, int nt,
-                                  const StepRef ts, float scaler, float *__restrict__ v) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if(k >= n) return;
-  const int t = step_index(ts);
-  v[k] = t >= 0 && t < nt ? traces[(size_t)t * nrt + rrid[k]] * scaler : 0.f;
+// The z kernel of a workgroup's columns, T[i] (in LDS) at plane cell cell(i), i < n:
+//   w0[col, offz+k] += T*kz[k]*vel, then with a mirror w0[col, 2*izm - (offz+k)] -= T*kz[k]*vel there
+// (distinct k of a column mirror to distinct cells; the direct terms of the workgroup's columns are complete).
+// Consecutive lanes take consecutive z of a column; five terms per lane are in flight: all of 64 columns' for the
+// usual 20-sample z kernels.
+template<class Cell>
+__device__ __forceinline__ void apply_columns(const GroupArgs &a, const float *T, int n, const Cell &cell,
+                                              const float *__restrict__ kz, float *w0, const float *__restrict__ vel) {
+  constexpr int U = 5;
+  const int lz = a.lz, tot = n * lz, step = blockDim.x;
+  for(int pass = 0; pass < (a.izm >= 0 ? 2 : 1); pass++) {
+    if(pass) __syncthreads();
+    for(int e0 = threadIdx.x; e0 < tot; e0 += U * step) {
+      float w[U], v[U], q[U];
+      size_t o[U];
+      bool ok[U];
+#pragma unroll
+      for(int u = 0; u < U; u++) {
+        const int e = e0 + u * step, ec = min(e, tot - 1), i = (int)((unsigned)ec / (unsigned)lz), k = ec - i * lz;
+        const int c = cell(i), py = (int)((unsigned)c / (unsigned)a.bw), px = c - py * a.bw;
+        const int iz = pass ? 2 * a.izm - (a.offz + k) : a.offz + k;
+        const float t = T[i];
+        ok[u] = e < tot && t != 0.f && iz >= 0 && iz < a.nz;
+        o[u] = ((size_t)(a.by0 + py) * a.nx + a.bx0 + px) * a.nz + (ok[u] ? iz : 0);
+        q[u] = t * kz[k];
+        w[u] = w0[o[u]], v[u] = vel[o[u]];
+      }
+#pragma unroll
+      for(int u = 0; u < U; u++)
+        if(ok[u]) w0[o[u]] = pass ? w[u] - q[u] * v[u] : w[u] + q[u] * v[u];
+    }
+  }
 }
-// X[j][px] = sum over receivers k of row j whose x kernel covers the cell of v[k]*kx_k (receivers in x-origin
-// order; an origin bin is clamped into the box, so each term is kept only where its tap index is in range)
-__global__ void inject_row_kernel(const GroupArgs a, int nrows, const int *__restrict__ rbin, const int *__restrict__ rorg,
-                                  const float *__restrict__ rkx, const float *__restrict__ v, float *__restrict__ X) {
+
+// Gather injection in one launch: 64 plane cells per workgroup, their sums, then their columns.  A source is a
+// few hundred cells, where launches are all that counts (factor, plane and apply kernels 12 us, this one 7).
+template<bool WY>
+__global__ void __launch_bounds__(256)
+    inject_gather_kernel(const GroupArgs a, const GatherTabs g, const TraceArgs tr, const float *__restrict__ kz, float *w0,
+                         const float *__restrict__ vel) {
+  __shared__ float T[64];
+  const int c0 = blockIdx.x * 64, i = threadIdx.x / IG, sub = threadIdx.x % IG;
+  const float t = gather_cell<WY>(a, g, tr, c0 + i, sub);
+  if(sub == 0) T[i] = t;
+  __syncthreads();
+  apply_columns(a, T, min(64, a.bw * a.bh - c0), [&](int j) { return c0 + j; }, kz, w0, vel);
+}
+
+// Separable form of the same plane.
+// X[j][px] = sum over receivers k of row j whose x kernel covers the cell of (val_k*scaler)*kx_k (receivers in
+// x-origin order; an origin bin is clamped into the box, so each term is kept only where its tap index is in
+// range).  Loads of SU terms go out together: the loop is a chain of load latencies otherwise (160 000 stations on
+// 400^2 cells: values + rows + columns + apply kernels 53 us, now rows 9 us + columns 20 us; the columns move
+// 0.10 GB, lines of which the 20 samples are less than half).
+constexpr int SU = 10;
+__global__ void __launch_bounds__(256)
+    inject_row_kernel(const GroupArgs a, int nrows, const int *__restrict__ rbin, const int *__restrict__ rorg,
+                      const int *__restrict__ rrid, const float *__restrict__ rkx, const TraceArgs tr,
+                      float *__restrict__ X) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= (long)nrows * a.bw) return;
   const int j = (int)(i / a.bw), px = (int)(i % a.bw), jx = a.bx0 + px, L = a.L;
+  const int t = step_index(tr.ts);
+  const bool on = t >= 0 && t < tr.nt;
+  const float *row = tr.traces + (size_t)(on ? t : 0) * tr.nrt;
   const int *b = rbin + (size_t)j * (a.bw + 1);
-  const int k0 = b[max(0, px - a.lxmax + 1)], k1 = b[px + 1];
+  const int k0 = b[max(0, px - a.lxmax + 1)], k1 = on ? b[px + 1] : 0;
   float s = 0.f;
-  for(int k = k0; k < k1; k++) {
-    const int ex = jx - rorg[k];
-    const float term = v[k] * rkx[(size_t)min(max(ex, 0), L - 1) * a.nr + k];
-    s += ex >= 0 && ex < L ? term : 0.f;
+  for(int kb = k0; kb < k1; kb += SU) {
+    int ex[SU];
+    float v[SU], x[SU];
+#pragma unroll
+    for(int u = 0; u < SU; u++) {
+      const int k = min(kb + u, k1 - 1);
+      ex[u] = jx - rorg[k];
+      v[u] = row[rrid[k]];
+    }
+#pragma unroll
+    for(int u = 0; u < SU; u++) x[u] = rkx[(size_t)min(max(ex[u], 0), L - 1) * a.nr + min(kb + u, k1 - 1)];
+#pragma unroll
+    for(int u = 0; u < SU; u++) {
+      const float term = (v[u] * tr.scaler) * x[u];
+      s += kb + u < k1 && ex[u] >= 0 && ex[u] < L ? term : 0.f;
+    }
   }
   X[i] = s;
 }
-// T[py][px] = sum over rows j whose y kernel covers the cell of ky_j*X[j][px] (rows in y-origin order)
-__global__ void inject_col_kernel(const GroupArgs a, int nrows, const int *__restrict__ cbin, const int *__restrict__ roy,
-                                  const float *__restrict__ rky, const float *__restrict__ X, float *__restrict__ plane) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if(c >= a.bw * a.bh) return;
-  const int px = c % a.bw, py = c / a.bw, jy = a.by0 + py, L = a.L;
-  const int j0 = cbin[max(0, py - a.lymax + 1)], j1 = cbin[py + 1];
-  float s = 0.f;
-  for(int j = j0; j < j1; j++) {
-    const int ey = jy - roy[j];
-    const float term = rky[(size_t)min(max(ey, 0), L - 1) * nrows + j] * X[(size_t)j * a.bw + px];
-    s += ey >= 0 && ey < L ? term : 0.f;
+// T[py][px] = sum over rows j whose y kernel covers the cell of ky_j*X[j][px] (rows in y-origin order), then the
+// z kernel of the columns: a workgroup owns 64 cells of ROWS plane rows, one row summed per wave
+template<int ROWS>
+__global__ void __launch_bounds__(256)
+    inject_col_kernel(const GroupArgs a, int nrows, const int *__restrict__ cbin, const int *__restrict__ roy,
+                      const float *__restrict__ rky, const float *__restrict__ X, const float *__restrict__ kz, float *w0,
+                      const float *__restrict__ vel) {
+  __shared__ float T[ROWS * 64];
+  const int nbx = (a.bw + 63) / 64, by = blockIdx.x / nbx, x0 = (blockIdx.x - by * nbx) * 64, y0 = by * ROWS;
+  const int py = y0 + (threadIdx.x >> 6), px = x0 + (threadIdx.x & 63);
+  if(threadIdx.x < ROWS * 64 && px < a.bw && py < a.bh) {
+    const int j0 = cbin[max(0, py - a.lymax + 1)], j1 = cbin[py + 1], jy = a.by0 + py, L = a.L;
+    float s = 0.f;
+    for(int jb = j0; jb < j1; jb += SU) {
+      int ey[SU];
+      float x[SU], y[SU];
+#pragma unroll
+      for(int u = 0; u < SU; u++) {
+        const int j = min(jb + u, j1 - 1);
+        ey[u] = jy - roy[j];
+        x[u] = X[(size_t)j * a.bw + px];
+      }
+#pragma unroll
+      for(int u = 0; u < SU; u++) y[u] = rky[(size_t)min(max(ey[u], 0), L - 1) * nrows + min(jb + u, j1 - 1)];
+#pragma unroll
+      for(int u = 0; u < SU; u++) {
+        const float term = y[u] * x[u];
+        s += jb + u < j1 && ey[u] >= 0 && ey[u] < L ? term : 0.f;
+      }
+    }
+    T[threadIdx.x] = s;
   }
-  plane[c] = s;
-}
-
-// w0[col, offz+k] += T*kz[k]*vel
-__global__ void inject_apply_kernel(const GroupArgs a, const float *__restrict__ plane, const float *__restrict__ kz,
-                                    float *__restrict__ w0, const float *__restrict__ vel) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long tot = (long)a.bw * a.bh * a.lz;
-  if(i >= tot) return;
-  int k = (int)(i % a.lz);
-  int c = (int)(i / a.lz);
-  int ix = a.bx0 + c % a.bw, iy = a.by0 + c / a.bw;
-  float T = plane[c];
-  if(T == 0.f) return;
-  size_t o = ((size_t)iy * a.nx + ix) * a.nz + a.offz + k;
-  w0[o] += (T * kz[k]) * vel[o];
-}
-
-// w0[col, 2*izm - (offz+k)] -= T*kz[k]*vel there (one lane per term; distinct k of a column mirror to
-// distinct cells)
-__global__ void inject_mirror_kernel(const GroupArgs a, const float *__restrict__ plane, const float *__restrict__ kz,
-                                     float *__restrict__ w0, const float *__restrict__ vel) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long tot = (long)a.bw * a.bh * a.lz;
-  if(i >= tot) return;
-  int k = (int)(i % a.lz);
-  int c = (int)(i / a.lz);
-  const int zm = 2 * a.izm - (a.offz + k);
-  if(zm < 0 || zm >= a.nz) return;
-  int ix = a.bx0 + c % a.bw, iy = a.by0 + c / a.bw;
-  float T = plane[c];
-  if(T == 0.f) return;
-  size_t o = ((size_t)iy * a.nx + ix) * a.nz + zm;
-  w0[o] -= (T * kz[k]) * vel[o];
+  __syncthreads();
+  for(int r = 0; r < ROWS && y0 + r < a.bh; r++)
+    apply_columns(a, T + 64 * r, min(64, a.bw - x0), [&](int i) { return (y0 + r) * a.bw + x0 + i; }, kz, w0, vel);
 }
 
 // P[iy][ix] = sum_k kz[k]*w[col, offz+k]
-__global__ void extract_plane_kernel(const GroupArgs a, const float *__restrict__ kz, const float *__restrict__ w,
-                                     float *__restrict__ plane) {
+__global__ void __launch_bounds__(256) extract_plane_kernel(const GroupArgs a, const float *__restrict__ kz,
+                                                            const float *__restrict__ w, float *__restrict__ plane) {
   int c = blockIdx.x * blockDim.x + threadIdx.x;
   if(c >= a.bw * a.bh) return;
   int ix = a.bx0 + c % a.bw, iy = a.by0 + c / a.bw;
   const float *col = w + ((size_t)iy * a.nx + ix) * a.nz + a.offz;
   float s = 0.f;
-  for(int k = 0; k < a.lz; k++) s += kz[k] * col[k];
+  for(int kb = 0; kb < a.lz; kb += SU) {
+    float v[SU];
+#pragma unroll
+    for(int u = 0; u < SU; u++) v[u] = col[min(kb + u, a.lz - 1)];
+#pragma unroll
+    for(int u = 0; u < SU; u++)
+      if(kb + u < a.lz) s += kz[kb + u] * v[u];
+  }
   if(a.izm >= 0) {
     // mirrored samples 2*izm - offz - k for k < lz2 = min(lz, 2*izm - offz + 1), inside the grid
     const float *colm = w + ((size_t)iy * a.nx + ix) * a.nz;
@@ -335,11 +408,19 @@ __global__ void extract_ycol_kernel(const GroupArgs a, int nrows, const int *__r
   const int j = (int)(i / a.bw), px = (int)(i % a.bw), L = a.L;
   const int y0 = roy[j] - a.by0;
   float s = 0.f;
-  for(int t = 0; t < L; t++) {
-    const int py = y0 + t;
-    const bool ok = py >= 0 && py < a.bh;
-    const float term = rky[(size_t)t * nrows + j] * plane[(size_t)min(max(py, 0), a.bh - 1) * a.bw + px];
-    s += ok ? term : 0.f;
+  for(int tb = 0; tb < L; tb += SU) {
+    float k[SU], p[SU];
+#pragma unroll
+    for(int u = 0; u < SU; u++) {
+      const int t = min(tb + u, L - 1);
+      k[u] = rky[(size_t)t * nrows + j], p[u] = plane[(size_t)min(max(y0 + t, 0), a.bh - 1) * a.bw + px];
+    }
+#pragma unroll
+    for(int u = 0; u < SU; u++) {
+      const int py = y0 + tb + u;
+      const float term = k[u] * p[u];
+      s += tb + u < L && py >= 0 && py < a.bh ? term : 0.f;
+    }
   }
   Z[i] = s;
 }
@@ -351,15 +432,26 @@ __global__ void extract_xrow_kernel(const GroupArgs a, const int *__restrict__ r
   const int L = a.L, x0 = rorg[k] - a.bx0;
   const float *z = Z + (size_t)rrow[k] * a.bw;
   float s = 0.f;
-  for(int t = 0; t < L; t++) {
-    const int px = x0 + t;
-    const bool ok = px >= 0 && px < a.bw;
-    const float term = rkx[(size_t)t * a.nr + k] * z[min(max(px, 0), a.bw - 1)];
-    s += ok ? term : 0.f;
+  for(int tb = 0; tb < L; tb += SU) {
+    float kx[SU], p[SU];
+#pragma unroll
+    for(int u = 0; u < SU; u++) {
+      const int t = min(tb + u, L - 1);
+      kx[u] = rkx[(size_t)t * a.nr + k], p[u] = z[min(max(x0 + t, 0), a.bw - 1)];
+    }
+#pragma unroll
+    for(int u = 0; u < SU; u++) {
+      const int px = x0 + tb + u;
+      const float term = kx[u] * p[u];
+      s += tb + u < L && px >= 0 && px < a.bw ? term : 0.f;
+    }
   }
   rec_row[rrid[k]] = s;
 }
 
+static GatherTabs gather_tabs(const Receiver &R, const RcvGroup &g) {
+  return GatherTabs{g.bin_start, g.bin_rcv, g.corg, g.ckx, g.cky, R.d_wy};
+}
 static GroupArgs gargs(const Receiver &R, const RcvGroup &g) {
   GroupArgs a;
   a.nx = R.nx, a.ny = R.ny, a.nz = R.nz, a.nr = g.nr;
@@ -494,10 +586,11 @@ int receiver_fk_spread(Receiver &R, float dx, float dy, float dt, int ntfft, flo
     for(auto &g : R.groups) {
       GroupArgs a = gargs(R, g);
       const int cells = g.bw * g.bh, nwy = g.nr * R.L;
-      hipLaunchKernelGGL(inject_wy_kernel, dim3(div_up(nwy, 256)), dim3(256), 0, stream(), nwy, g.nr, g.bin_rcv, g.cky,
-                         R.d_traces, R.nr, R.nt, ts, 1.0f, R.d_wy);
-      hipLaunchKernelGGL(inject_plane_kernel<IG>, dim3(div_up((long)cells * IG, 256)), dim3(256), 0, stream(), a,
-                         g.bin_start, g.corg, g.ckx, R.d_wy, R.d_plane);
+      const TraceArgs tr{R.d_traces, R.nr, R.nt, ts, 1.0f};
+      hipLaunchKernelGGL(inject_wy_kernel, dim3(div_up(nwy, 256)), dim3(256), 0, stream(), nwy, g.nr, g.bin_rcv, g.cky, tr,
+                         R.d_wy);
+      hipLaunchKernelGGL(inject_plane_kernel, dim3(div_up((long)cells * IG, 256)), dim3(256), 0, stream(), a,
+                         gather_tabs(R, g), tr, R.d_plane);
       hipLaunchKernelGGL(fk_gather_kernel, dim3(div_up(cells, 256)), dim3(256), 0, stream(), R.d_plane, data, g.bx0, g.by0,
                          g.bw, g.bh, nx, ntfft, it);
     }
@@ -584,29 +677,36 @@ int receiver_apply_at(Receiver &R, float *w0, const StepRef &ts, const float *ve
     return check_launch("fk_apply_kernel");
   }
   LaunchTimer tm("inject");
+  const TraceArgs tr{R.d_traces, R.nr, R.nt, ts, scaler};
   for(auto &g : R.groups) {
     GroupArgs a = gargs(R, g);
+    a.izm = iz_mirror;
     int cells = g.bw * g.bh;
     if(g.sep) {  // rows' x spreads, then their y spread (about 2 * 2 * spread terms per cell)
-      hipLaunchKernelGGL(inject_val_kernel, dim3(div_up(g.nr, 256)), dim3(256), 0, stream(), g.nr, g.rrid, R.d_traces,
-                         R.nr, R.nt, ts, scaler, R.d_wy);
       const long nrow = (long)g.nrows * g.bw;
       hipLaunchKernelGGL(inject_row_kernel, dim3(div_up(nrow, 256)), dim3(256), 0, stream(), a, g.nrows, g.rbin, g.rorg,
-                         g.rkx, R.d_wy, R.d_rows);
-      hipLaunchKernelGGL(inject_col_kernel, dim3(div_up(cells, 256)), dim3(256), 0, stream(), a, g.nrows, g.cbin, g.roy,
-                         g.rky, R.d_rows, R.d_plane);
+                         g.rrid, g.rkx, tr, R.d_rows);
+      // four rows a workgroup once that still fills the chip (400^2: 22.5 us, one row 26); one row below, where
+      // the walk down the columns is what a workgroup takes (128^2: 6.3 us, four rows 11)
+      if(cells >= 65536)
+        hipLaunchKernelGGL(inject_col_kernel<4>, dim3(div_up(g.bw, 64) * div_up(g.bh, 4)), dim3(256), 0, stream(), a, g.nrows,
+                           g.cbin, g.roy, g.rky, R.d_rows, g.kz, w0, vel);
+      else
+        hipLaunchKernelGGL(inject_col_kernel<1>, dim3(div_up(g.bw, 64) * g.bh), dim3(256), 0, stream(), a, g.nrows, g.cbin,
+                           g.roy, g.rky, R.d_rows, g.kz, w0, vel);
+      continue;
+    }
+    const GatherTabs tabs = gather_tabs(R, g);
+    // the y factors of a few receivers are formed where they are used; many receivers reach a cell hundreds of
+    // times, where a factor read from memory beats two dependent loads
+    if(g.nr <= 4096) {
+      hipLaunchKernelGGL(inject_gather_kernel<false>, dim3(div_up(cells, 64)), dim3(256), 0, stream(), a, tabs, tr, g.kz, w0,
+                         vel);
     } else {
       const int nw = g.nr * R.L;
-      hipLaunchKernelGGL(inject_wy_kernel, dim3(div_up(nw, 256)), dim3(256), 0, stream(), nw, g.nr, g.bin_rcv, g.cky,
-                         R.d_traces, R.nr, R.nt, ts, scaler, R.d_wy);
-      hipLaunchKernelGGL(inject_plane_kernel<IG>, dim3(div_up((long)cells * IG, 256)), dim3(256), 0, stream(), a,
-                         g.bin_start, g.corg, g.ckx, R.d_wy, R.d_plane);
-    }
-    long tot = (long)cells * g.lz;
-    hipLaunchKernelGGL(inject_apply_kernel, dim3(div_up(tot, 256)), dim3(256), 0, stream(), a, R.d_plane, g.kz, w0, vel);
-    if(iz_mirror >= 0) {
-      a.izm = iz_mirror;
-      hipLaunchKernelGGL(inject_mirror_kernel, dim3(div_up(tot, 256)), dim3(256), 0, stream(), a, R.d_plane, g.kz, w0,
+      hipLaunchKernelGGL(inject_wy_kernel, dim3(div_up(nw, 256)), dim3(256), 0, stream(), nw, g.nr, g.bin_rcv, g.cky, tr,
+                         R.d_wy);
+      hipLaunchKernelGGL(inject_gather_kernel<true>, dim3(div_up(cells, 64)), dim3(256), 0, stream(), a, tabs, tr, g.kz, w0,
                          vel);
     }
   }
