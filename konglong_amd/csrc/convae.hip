@@ -24,7 +24,8 @@
 // output channels (padded), K = 27 taps x gathered channels, the A operand
 // gathered from the input tensor per tap (im2col on the fly, zero outside the
 // grid), the B operand from weights pre-arranged in fragment order after every
-// update.  Weight gradient: M = 32 output channels, N = 32 (tap, input channel)
+// update; the upsampling layers' and the output layer's forward have kernels of
+// their own (cae_up_kernel, cae_last_kernel).  Weight gradient: M = 32 output channels, N = 32 (tap, input channel)
 // pairs, K = positions, accumulated per wave and added with FP32 atomics.
 // Training minimises the mean squared reconstruction error with Adam.
 #include "klrtm_internal.h"
@@ -149,6 +150,207 @@ __global__ void __launch_bounds__(256) cae_conv_kernel(const float *__restrict__
       out[o] = v;
     }
   }
+}
+
+// ---- nearest x2 upsampling + 3x3x3 convolution, 32 -> COUT channels -----------------------------------
+//
+// A fine cell f = 2i + a (phase a in {0,1}^3) sees, along each axis, only the coarse cells i + t + a - 1, t in
+// {0,1}: the three taps of a phase fall on two coarse cells.  So a phase is a 2x2x2 convolution of the coarse grid
+// whose weights are sums of the layer's BF16-rounded weights.  A sum of up to eight is kept as two BF16 terms, its
+// rounding and the rest (2^-17 of it is lost; one rounded term moved a decoded volume by 0.8 %): 16 products a
+// phase instead of 27.
+// One workgroup owns TY x TX x Dc coarse cells, staged with their halo as BF16 in LDS (pitch 80 bytes a cell: the
+// 16 cells of a fragment read fall on distinct banks).  A wave takes the two phases of one (ay, ax) at a time, for 16
+// output channels, keeps their 32 weight fragments in registers while it walks the tile's cells, and reads each
+// coarse cell's fragment once for both: 12 LDS reads for 32 matrix products v_mfma_f32_16x16x32_bf16.
+// Operand layouts (lane l):
+//   A: A[l % 16][(l / 16)*8 + t]   B: B[(l / 16)*8 + t][l % 16]   C: register r holds C[(l / 16)*4 + r][l % 16]
+// 128 blocks: 161 us for layer 6 (about half of it the vector instructions of 67 M exact GELUs, 27 us the matrix
+// products, 268 MB written) and 42 us for layer 5; gathering 27 taps per fine cell from L2, as the other layers do,
+// the two took 1364 us.
+typedef float cae_f32x4 __attribute__((ext_vector_type(4)));
+constexpr int CAE_UP_TY = 2, CAE_UP_TX = 8, CAE_UP_PITCH = 80;
+
+template<int COUT, int LGD>
+__global__ void __launch_bounds__(256, 2) cae_up_kernel(const float *__restrict__ X, const cae_bf16x8 *__restrict__ wu,
+                                                        const float *__restrict__ bias, float *__restrict__ z,
+                                                        float *__restrict__ out) {
+  constexpr int Dc = 1 << LGD, Df = 2 * Dc, TY = CAE_UP_TY, TX = CAE_UP_TX;
+  constexpr int SZ = Dc + 2, SX = (TX + 2) * SZ, CELLS = (TY + 2) * SX;  // LDS strides in cells
+  constexpr int NXT = Dc / TX, NYT = Dc / TY;
+  __shared__ __attribute__((aligned(16))) char lds[CELLS * CAE_UP_PITCH];
+  const int tile = blockIdx.x, y0 = (tile / NXT) * TY, x0 = (tile % NXT) * TX;
+  static_assert(NYT * TY == Dc && NXT * TX == Dc, "whole tiles");
+  const size_t b = blockIdx.y;
+  const float *Xb = X + b * ((size_t)32 << (3 * LGD));
+  // stage the tile: four channels per thread and step
+  for(int e = threadIdx.x; e < CELLS * 8; e += 256) {
+    const int cell = e >> 3, c4 = (e & 7) * 4;
+    const int ly = cell / SX, r = cell - ly * SX, lx = r / SZ, lz = r - lx * SZ;
+    const int y = y0 + ly - 1, x = x0 + lx - 1, zz = lz - 1;
+    float4 v = {0.f, 0.f, 0.f, 0.f};
+    if((unsigned)y < (unsigned)Dc && (unsigned)x < (unsigned)Dc && (unsigned)zz < (unsigned)Dc)
+      v = *(const float4 *)(Xb + (size_t)(((y << LGD) + x) << LGD) * 32 + zz * 32 + c4);
+    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+    bf4 h;
+    h[0] = (__bf16)v.x, h[1] = (__bf16)v.y, h[2] = (__bf16)v.z, h[3] = (__bf16)v.w;
+    *(bf4 *)(lds + cell * CAE_UP_PITCH + c4 * 2) = h;
+  }
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, n = lane & 15;
+  // two passes: COUT 32: wave = (ay, ax), pass = half of the channels; COUT 16: wave = (ay, every second row of
+  // cells), pass = ax
+  constexpr int NT = COUT / 16, RPM = Dc == 8 ? 2 : 1, MT = TY * TX / RPM;  // 16 cells: one row of 16 or two of 8
+  __syncthreads();
+  for(int pass = 0; pass < 2; pass++) {
+    const int ay = COUT == 32 ? w >> 1 : w & 1, ax = COUT == 32 ? w & 1 : pass, h = COUT == 32 ? pass : 0;
+    cae_bf16x8 B[2][8][2];  // [az][t][rounded, rest]
+#pragma unroll
+    for(int az = 0; az < 2; az++)
+#pragma unroll
+      for(int t = 0; t < 8; t++)
+#pragma unroll
+        for(int k = 0; k < 2; k++) B[az][t][k] = wu[(((((ay * 2 + ax) * 2 + az) * 8 + t) * NT + h) * 2 + k) * 64 + lane];
+    const float bn = bias[h * 16 + n];
+    for(int m = COUT == 32 ? 0 : w >> 1; m < MT; m += COUT == 32 ? 1 : 2) {
+      const int row = m * RPM + (Dc == 8 ? n >> 3 : 0), ly = row / TX, lx = row % TX, lz = n & (Dc - 1);
+      const char *base = lds + ((ly + ay) * SX + (lx + ax) * SZ + lz) * CAE_UP_PITCH + q * 16;
+      cae_f32x4 acc[2] = {};
+#pragma unroll
+      for(int ty = 0; ty < 2; ty++)
+#pragma unroll
+        for(int tx = 0; tx < 2; tx++)
+#pragma unroll
+          for(int oz = 0; oz < 3; oz++) {  // coarse z offset oz - 1: tap oz - az of phase az
+            const cae_bf16x8 a = *(const cae_bf16x8 *)(base + (ty * SX + tx * SZ + oz) * CAE_UP_PITCH);
+#pragma unroll
+            for(int az = 0; az < 2; az++) {
+              if(oz - az < 0 || oz - az > 1) continue;
+#pragma unroll
+              for(int k = 0; k < 2; k++)
+                acc[az] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, B[az][(ty * 2 + tx) * 2 + oz - az][k], acc[az], 0, 0, 0);
+            }
+          }
+#pragma unroll
+      for(int r = 0; r < 4; r++) {
+        const int mr = q * 4 + r, rr = m * RPM + (Dc == 8 ? mr >> 3 : 0);
+        const int cy = y0 + rr / TX, cx = x0 + rr % TX, cz = mr & (Dc - 1);
+#pragma unroll
+        for(int az = 0; az < 2; az++) {
+          const size_t f = ((size_t)(2 * cy + ay) * Df + (2 * cx + ax)) * Df + (2 * cz + az);
+          const size_t o = (b * ((size_t)1 << (3 * LGD + 3)) + f) * COUT + h * 16 + n;
+          const float v = acc[az][r] + bn;
+          if(z) z[o] = v;
+          out[o] = gelu(v);
+        }
+      }
+    }
+  }
+}
+
+// phase fragments of an upsampling layer: wu[((ay, ax, az), (ty, tx, tz), half, rounded / rest)][lane], k = input
+// channel
+__global__ void cae_wup_kernel(const float *__restrict__ W, int cout, cae_bf16x8 *__restrict__ wu) {
+  const int nt = cout / 16, i = blockIdx.x * blockDim.x + threadIdx.x;
+  if(i >= 64 * nt * 64) return;
+  const int l = i & 63, h = (i >> 6) % nt, t = (i >> 6) / nt % 8, a = (i >> 6) / nt / 8;
+  const int co = h * 16 + (l & 15);
+  // taps d (0..2 for -1..1) of phase bit p that fall on coarse offset t + p - 1: p = 0: {0}, {1, 2}; p = 1: {0, 1}, {2}
+  auto lo = [](int p, int tt) { return tt == 0 ? 0 : p == 0 ? 1 : 2; };
+  auto hi = [](int p, int tt) { return tt == 1 ? 2 : p == 0 ? 0 : 1; };
+  const int ay = a >> 2, ax = (a >> 1) & 1, az = a & 1, ty = t >> 2, tx = (t >> 1) & 1, tz = t & 1;
+  cae_bf16x8 v, r;
+#pragma unroll
+  for(int j = 0; j < 8; j++) {
+    const int ci = (l >> 4) * 8 + j;
+    float s = 0.f;
+    for(int dy = lo(ay, ty); dy <= hi(ay, ty); dy++)
+      for(int dx = lo(ax, tx); dx <= hi(ax, tx); dx++)
+        for(int dz = lo(az, tz); dz <= hi(az, tz); dz++) s += (float)(__bf16)W[((size_t)co * 32 + ci) * 27 + (dy * 3 + dx) * 3 + dz];
+    v[j] = (__bf16)s;
+    r[j] = (__bf16)(s - (float)v[j]);
+  }
+  const size_t o = ((size_t)(i >> 6) * 2) * 64 + l;
+  wu[o] = v, wu[o + 64] = r;
+}
+
+// ---- the output layer: 3x3x3 convolution of 16 channels to one on the 32^3 grid ------------------------
+//
+// First the products of every cell with all 27 taps, T[cell][tap] = sum_c x[cell][c] W[tap][c] (one
+// v_mfma_f32_32x32x16_bf16 per row of 32 cells: taps are the columns), then y[p] = sum_tap T[p + d(tap)][tap] from LDS.
+// As an ordinary implicit GEMM one of 32 columns did useful work and every cell's channels were gathered 27 times
+// (513 us for 128 blocks, now 58 us).  A workgroup owns 8 rows (and one more on each side) and walks along y; each thread keeps
+// the three output planes its cell contributes to.
+__global__ void cae_wtap_kernel(const float *__restrict__ W, cae_bf16x8 *__restrict__ wt) {
+  const int l = threadIdx.x, tap = l & 31;
+  cae_bf16x8 v;
+#pragma unroll
+  for(int j = 0; j < 8; j++) v[j] = (__bf16)(tap < 27 ? W[((l >> 5) * 8 + j) * 27 + tap] : 0.f);
+  wt[l] = v;
+}
+__global__ void __launch_bounds__(256) cae_last_kernel(const float *__restrict__ X, const cae_bf16x8 *__restrict__ wt,
+                                                       const float *__restrict__ bias, float *__restrict__ out) {
+  constexpr int ROWS = 10;
+  __shared__ float T[ROWS * 32 * 27];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int x0 = blockIdx.x * 8;
+  const size_t b = blockIdx.y;
+  const float *Xb = X + b * (32768 * 16);
+  const cae_bf16x8 B = wt[lane];
+  const int lx = threadIdx.x >> 5, lz = threadIdx.x & 31;  // this thread's output column
+  float o0 = bias[0], o1 = o0, o2;  // outputs of planes y-1, y, y+1
+  // rows w, w + 4, w + 8 of plane y
+  auto load = [&](int y, float4(&v)[3][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for(int k = 0; k < 3; k++) {
+      const int r = w + 4 * k, x = x0 + r - 1;
+      v[k][0] = v[k][1] = float4{0.f, 0.f, 0.f, 0.f};
+      if(r < ROWS && (unsigned)x < 32u && y < 32) {
+        const float4 *src = (const float4 *)(Xb + (((size_t)y * 32 + x) * 32 + (lane & 31)) * 16 + (lane >> 5) * 8);
+        v[k][0] = src[0], v[k][1] = src[1];
+      }
+    }
+  };
+  float4 v[3][2];
+  load(0, v);
+  for(int y = 0; y < 32; y++) {
+    cae_f32x16 acc[3];
+#pragma unroll
+    for(int k = 0; k < 3; k++) {
+      cae_bf16x8 a;
+      a[0] = (__bf16)v[k][0].x, a[1] = (__bf16)v[k][0].y, a[2] = (__bf16)v[k][0].z, a[3] = (__bf16)v[k][0].w;
+      a[4] = (__bf16)v[k][1].x, a[5] = (__bf16)v[k][1].y, a[6] = (__bf16)v[k][1].z, a[7] = (__bf16)v[k][1].w;
+      acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B, cae_f32x16{}, 0, 0, 0);
+    }
+    load(y + 1, v);
+    __syncthreads();  // the sums of plane y-1 are done with T
+    const int tap = lane & 31;
+    if(tap < 27) {
+#pragma unroll
+      for(int k = 0; k < 3; k++)
+        if(w + 4 * k < ROWS) {
+#pragma unroll
+          for(int r = 0; r < 16; r++)
+            T[((w + 4 * k) * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * 27 + tap] = acc[k][r];
+        }
+    }
+    __syncthreads();
+    // y[p] += T[p + d][tap(d)]: plane y is d_y = +1 of output y-1, 0 of y, -1 of y+1
+    float s[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for(int dx = 0; dx < 3; dx++)
+#pragma unroll
+      for(int dz = 0; dz < 3; dz++) {
+        const int zz = lz + dz - 1;
+        const float *t = T + ((lx + dx) * 32 + min(max(zz, 0), 31)) * 27 + dx * 3 + dz;
+        const bool ok = (unsigned)zz < 32u;
+#pragma unroll
+        for(int dy = 0; dy < 3; dy++) s[dy] += ok ? t[dy * 9] : 0.f;
+      }
+    o0 += s[2], o1 += s[1], o2 = bias[0] + s[0];
+    if(y > 0) out[b * 32768 + ((size_t)(y - 1) * 32 + x0 + lx) * 32 + lz] = o0;
+    o0 = o1, o1 = o2;
+  }
+  out[b * 32768 + ((size_t)31 * 32 + x0 + lx) * 32 + lz] = o0;
 }
 
 // dW[co][ci][tap] += sum_{b, p} dZ[b][p][co] * X[b][q(p, tap)][ci] over a chunk of CAE_WG_CHUNK positions of
@@ -426,6 +628,8 @@ static int lg2(int d) {
   return l;
 }
 static int ksteps(int ch) { return (ch * 27 + 15) / 16; }
+// the upsampling layers and the output layer have fragments of their own for the forward pass
+static int fwd_ksteps(int l) { return kKind[l] == K_UP || l == CAE_LAYERS - 1 ? 0 : ksteps(kCin[l]); }
 
 CaeWork::~CaeWork() {
   for(int l = 0; l < CAE_LAYERS; l++) (void)hipFree(z[l]), (void)hipFree(a[l]);
@@ -435,6 +639,7 @@ CaeWork::~CaeWork() {
 
 ConvAE::~ConvAE() {
   for(void *p : {(void *)d_param, (void *)d_grad, (void *)d_m, (void *)d_v, d_wf, d_wb, (void *)d_loss}) (void)hipFree(p);
+  for(void *p : d_wu) (void)hipFree(p);
 }
 
 size_t cae_param_count() {
@@ -452,7 +657,7 @@ int cae_create(ConvAE **out, unsigned seed) {
     c->b_off[l] = off;
     off += kCout[l];
     c->wf_off[l] = foff, c->wb_off[l] = boff;
-    foff += (size_t)ksteps(kCin[l]) * 64;
+    foff += (size_t)fwd_ksteps(l) * 64;
     boff += (size_t)ksteps(kCout[l]) * 64;
   }
   c->nparam = off;
@@ -471,6 +676,9 @@ int cae_create(ConvAE **out, unsigned seed) {
   if(e == hipSuccess) e = hipMalloc(&c->d_v, off * 4);
   if(e == hipSuccess) e = hipMalloc(&c->d_wf, foff * sizeof(cae_bf16x8));
   if(e == hipSuccess) e = hipMalloc(&c->d_wb, boff * sizeof(cae_bf16x8));
+  for(int l = 0; l < CAE_LAYERS && e == hipSuccess; l++)
+    if(kKind[l] == K_UP) e = hipMalloc(&c->d_wu[l], (size_t)64 * (kCout[l] / 16) * 2 * 64 * sizeof(cae_bf16x8));
+    else if(l == CAE_LAYERS - 1) e = hipMalloc(&c->d_wu[l], 64 * sizeof(cae_bf16x8));
   if(e == hipSuccess) e = hipMalloc(&c->d_loss, sizeof(float) * 2);
   if(e == hipSuccess) e = hipMemcpy(c->d_param, h.data(), off * 4, hipMemcpyHostToDevice);
   if(e == hipSuccess) e = hipMemset(c->d_m, 0, off * 4);
@@ -492,9 +700,14 @@ int cae_create(ConvAE **out, unsigned seed) {
 // weight fragments from the FP32 weights
 int cae_refresh(ConvAE &c) {
   for(int l = 0; l < CAE_LAYERS; l++) {
-    const int ksf = ksteps(kCin[l]), ksb = ksteps(kCout[l]), n = (ksf + ksb) * 64;
+    const int ksf = fwd_ksteps(l), ksb = ksteps(kCout[l]), n = (ksf + ksb) * 64;
     hipLaunchKernelGGL(cae_wfrag_kernel, dim3((n + 255) / 256), dim3(256), 0, stream(), c.d_param + c.w_off[l], kCin[l],
                        kCout[l], ksf, ksb, (cae_bf16x8 *)c.d_wf + c.wf_off[l], (cae_bf16x8 *)c.d_wb + c.wb_off[l]);
+    if(kKind[l] == K_UP)
+      hipLaunchKernelGGL(cae_wup_kernel, dim3(kCout[l] / 16 * 16), dim3(256), 0, stream(), c.d_param + c.w_off[l], kCout[l],
+                         (cae_bf16x8 *)c.d_wu[l]);
+    else if(l == CAE_LAYERS - 1)
+      hipLaunchKernelGGL(cae_wtap_kernel, dim3(1), dim3(64), 0, stream(), c.d_param + c.w_off[l], (cae_bf16x8 *)c.d_wu[l]);
   }
   return check_launch("cae_wfrag_kernel");
 }
@@ -552,15 +765,31 @@ static int layer_fwd(const ConvAE &c, int l, const float *in, float *z, float *o
   const int lgo = lg2(kDout[l]), lgg = lg2(kDin[l]), ks = ksteps(kCin[l]);
   const void *wf = (const cae_bf16x8 *)c.d_wf + c.wf_off[l];
   const float *bias = c.d_param + c.b_off[l];
-  const int mode = kKind[l] == K_DOWN ? G_DOWN : kKind[l] == K_UP ? G_UP : G_SAME;
+  const cae_bf16x8 *wu = (const cae_bf16x8 *)c.d_wu[l];
+  if(kKind[l] == K_UP) {
+    const int tiles = (kDin[l] / CAE_UP_TY) * (kDin[l] / CAE_UP_TX);
+    const dim3 grid((unsigned)tiles, (unsigned)nb);
+    if(kCout[l] == 32 && kDin[l] == 8)
+      hipLaunchKernelGGL((cae_up_kernel<32, 3>), grid, dim3(256), 0, stream(), in, wu, bias, z, out);
+    else if(kCout[l] == 16 && kDin[l] == 16)
+      hipLaunchKernelGGL((cae_up_kernel<16, 4>), grid, dim3(256), 0, stream(), in, wu, bias, z, out);
+    else {
+      set_error("autoencoder layer %d has no forward kernel", l);
+      return KLRTM_EINVAL;
+    }
+    return check_launch("cae_up_kernel");
+  }
+  if(l == CAE_LAYERS - 1) {  // (no activation: nothing reads its pre-activation)
+    hipLaunchKernelGGL(cae_last_kernel, dim3(4, (unsigned)nb), dim3(256), 0, stream(), in, wu, bias, out);
+    return check_launch("cae_last_kernel");
+  }
+  const int mode = kKind[l] == K_DOWN ? G_DOWN : G_SAME;
 #define CAE_F(CG, M) conv_launch<CG, M, E_FWD>(in, wf, ks, kCout[l], lgo, lgg, bias, kGelu[l], z, out, nullptr, nb)
   switch(kCin[l] * 8 + mode) {
   case 1 * 8 + G_DOWN: CAE_F(1, G_DOWN); break;
   case 16 * 8 + G_DOWN: CAE_F(16, G_DOWN); break;
   case 32 * 8 + G_SAME: CAE_F(32, G_SAME); break;
   case 4 * 8 + G_SAME: CAE_F(4, G_SAME); break;
-  case 32 * 8 + G_UP: CAE_F(32, G_UP); break;
-  case 16 * 8 + G_SAME: CAE_F(16, G_SAME); break;
   default: set_error("autoencoder layer %d has no forward kernel", l); return KLRTM_EINVAL;
   }
 #undef CAE_F

@@ -1,0 +1,54 @@
+"""Upsampling and output layers of the autoencoder near the edges of their tiles.
+
+The upsampling layers are computed per output phase from the coarse grid in tiles of 2 x 8 x D cells, the
+output layer as sums over products with all taps in slabs of 8 rows: rough inputs and non-zero biases, so
+that every tap, phase, halo and tile boundary carries weight, for one block and for odd counts.
+
+Bounds: the device and the reference round the same operands to BF16, but their FP32 summation orders
+differ by about 1e-6, so now and then an operand falls on the other side of a rounding boundary and moves by
+one BF16 step, up to 2^-7 of itself.  In the last layer one such step moves an output by up to
+2^-7 max|a| max|W| (a: its inputs); four times that is left for steps of earlier layers and for several at
+once.  Steps are rare: over any one plane of cells the rms error stays under 2^-7 of the output's rms (27
+cells at the largest step seen, 2.8 % of the rms, are 0.5 % over a plane of 1024).  A dropped or misplaced
+tap of one cell is off by 1/sqrt(27) of the rms, and of one row of 32 cells by 3.4 % over the plane."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from konglong_amd._lib import DeviceArray, check, lib
+from tests import convae_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nb", [1, 2, 7])
+def test_every_cell_of_rough_blocks(klrtm, nb):
+    print(f"[convae] forward of {nb} rough blocks, cell by cell", flush=True)
+    h = C.c_void_p()
+    check(lib().klrtm_convae_create(C.byref(h), 21))
+    rng = np.random.default_rng(900 + nb)
+    p = np.empty(lib().klrtm_convae_param_count(), np.float32)
+    check(lib().klrtm_convae_get_params(h.value, p.ctypes.data))
+    o = 0
+    for ci, co in zip(ref.CIN, ref.COUT):
+        o += co * ci * 27
+        p[o:o + co] = rng.uniform(-0.3, 0.3, co)
+        o += co
+    check(lib().klrtm_convae_set_params(h.value, p.ctypes.data))
+    x = rng.standard_normal((nb, 32, 32, 32)).astype(np.float32)
+    dx, rec = DeviceArray.from_host(x), DeviceArray((nb, 32, 32, 32))
+    check(lib().klrtm_convae_forward(h.value, dx.ptr, nb, None, rec.ptr))
+    lib().klrtm_convae_destroy(h.value)
+    a7 = ref.forward(p, torch.from_numpy(x.reshape(nb, 1, 32, 32, 32)), l1=7)[0]
+    want = ref.forward(p, a7, l0=7)[0].numpy().reshape(nb, 32, 32, 32)
+    w7 = ref.split_params(p)[7][0]
+    rms = np.sqrt(np.mean(want.astype(np.float64) ** 2))
+    err = np.abs(rec.download().astype(np.float64) - want)
+    planes = [np.sqrt(np.mean(err ** 2, axis=tuple(i for i in range(1, 4) if i != ax))) for ax in (1, 2, 3)]
+    bound = 4.0 * 2.0 ** -7 * float(a7.abs().max()) * float(np.abs(w7).max())
+    print(f"[convae] largest error {err.max():.2e} (bound {bound:.2e}), of a plane {np.max(planes):.2e} (rms {rms:.2e})",
+          flush=True)
+    assert err.max() <= bound
+    assert np.max(planes) <= 2.0 ** -7 * rms
