@@ -13,6 +13,7 @@ struct CaeWork {
   bool train = false;
   float *z[CAE_LAYERS] = {}, *a[CAE_LAYERS] = {};
   float *g0 = nullptr, *g1 = nullptr, *g2 = nullptr, *x = nullptr, *scale = nullptr, *ss = nullptr, *part = nullptr;
+  float *wpart = nullptr;  // training: partial weight gradients
   void *org = nullptr;
   ~CaeWork();
 };

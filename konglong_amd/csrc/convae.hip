@@ -25,8 +25,10 @@
 // gathered from the input tensor per tap (im2col on the fly, zero outside the
 // grid), the B operand from weights pre-arranged in fragment order after every
 // update; the upsampling layers' and the output layer's forward have kernels of
-// their own (cae_up_kernel, cae_last_kernel).  Weight gradient: M = 32 output channels, N = 32 (tap, input channel)
-// pairs, K = positions, accumulated per wave and added with FP32 atomics.
+// their own (cae_up_kernel, cae_last_kernel).  Weight gradient: M = 32 output
+// channels, N = 32 (tap, input channel) pairs, K = positions, accumulated per
+// wave and added with FP32 atomics; the upsampling and the single-channel layers
+// again have their own (cae_wgrad_up_kernel, cae_wgrad_vec_kernel).
 // Training minimises the mean squared reconstruction error with Adam.
 #include "klrtm_internal.h"
 #include "convae.h"
@@ -52,14 +54,13 @@ static const int kGelu[CAE_LAYERS] = {1, 1, 1, 0, 1, 1, 1, 0};
 
 // gather modes of the implicit GEMM: the gathered-tensor cell q of output position p and tap offset d
 // (per axis), on grids of side Dout (GEMM output) and Dg (gathered tensor)
-enum { G_SAME = 0, G_DOWN = 1, G_UP = 2, G_BSAME = 3, G_BDOWN = 4 };
+enum { G_SAME = 0, G_DOWN = 1, G_BSAME = 2, G_BDOWN = 3 };
 
 __device__ __forceinline__ int gather1(int mode, int p, int d, int Dout, int Dg) {
   int q;
   switch(mode) {
   case G_SAME: q = p + d; break;                                   // y[p] += w[d] x[p + d]
   case G_DOWN: q = 2 * p + d; break;                               // y[p] += w[d] x[2p + d]
-  case G_UP: q = p + d; return q >= 0 && q < Dout ? q >> 1 : -1;   // y[p] += w[d] x[(p + d) / 2]
   case G_BSAME: q = p - d; break;                                  // dx[p] += w[d]^T dy[p - d]
   default: q = p - d; return q >= 0 && !(q & 1) && (q >> 1) < Dg ? q >> 1 : -1;  // dx[p] += w[d]^T dy[(p - d)/2]
   }
@@ -353,6 +354,225 @@ __global__ void __launch_bounds__(256) cae_last_kernel(const float *__restrict__
   out[b * 32768 + ((size_t)31 * 32 + x0 + lx) * 32 + lz] = o0;
 }
 
+// ---- weight gradients of the upsampling layers ---------------------------------------------------------
+//
+// dW[co][ci][d] = sum over phases a of G[a][t(a, d)][co][ci], where
+//   G[a][t][co][ci] = sum_i dZ[2i + a][co] X[i + t + a - 1][ci]
+// runs over coarse cells i: 64 products a coarse cell instead of 8 * 27, with the same BF16 operands and FP32 sums.
+// K = positions, so both operands lie in LDS as runs of 8 z positions of one channel: chunk[row][z / 8][channel],
+// X three times, shifted by -1, 0, +1 in z, dZ split by phase.  Rows of a fragment's 16 channels are 256 contiguous
+// bytes.  A workgroup walks tiles of TY x TX coarse rows; the next tile's loads are in flight during the products.
+// Wave = (ay, ax, half of the input channels): 16 accumulators, 14 LDS reads for 16 products.  blockIdx.y = 16 output
+// channels.  Sums of a workgroup go to its slot of `part`; cae_wred_kernel and cae_wup_sum_kernel add them in a fixed
+// order.
+constexpr int CAE_UPG = 64 * 16 * 32;  // products of one workgroup
+
+template<int COUT, int LGD>
+__global__ void __launch_bounds__(512) cae_wgrad_up_kernel(const float *__restrict__ X, const float *__restrict__ dZ,
+                                                           int ntask, float *__restrict__ part) {
+  constexpr int Dc = 1 << LGD, Df = 2 * Dc, NCH = Dc / 8, TY = 2, TX = Dc == 8 ? 4 : 2, SX = TX + 2;
+  constexpr int HROWS = (TY + 2) * SX, ROWS = TY * TX, KS = ROWS * NCH / 4, NXT = Dc / TX, TILES = NXT * (Dc / TY);
+  __shared__ __attribute__((aligned(16))) char xs[3 * HROWS * NCH * 32 * 16], zs[ROWS * 8 * NCH * 16 * 16];
+  typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+  const int tid = threadIdx.x, c0 = blockIdx.y * 16;
+  // staging: X, one chunk (with one cell more on both ends) of two channels; dZ, eight fine cells of two channels
+  const int xc = tid & 15, xch = (tid >> 4) % NCH, xrow = (tid >> 4) / NCH;
+  const int zc = tid & 7, zh = (tid >> 3) & 1, zch = (tid >> 4) % NCH, zph = (tid >> 4) / NCH & 3, zrow = (tid >> 4) / NCH >> 2;
+  static_assert(HROWS * NCH * 16 <= 512 && ROWS * 4 * NCH * 16 == 512, "one item per thread");
+  float2 xv[10], zv[8];
+  auto load = [&](int task) __attribute__((always_inline)) {
+    const size_t b = task / TILES;
+    const int tile = task % TILES, y0 = tile / NXT * TY, x0 = tile % NXT * TX;
+    const int y = y0 + xrow / SX - 1, x = x0 + xrow % SX - 1;
+    const bool in = xrow < HROWS && (unsigned)y < (unsigned)Dc && (unsigned)x < (unsigned)Dc;
+    const float *sx = X + ((b << (3 * LGD)) + (size_t)(((y << LGD) + x) << LGD) + xch * 8) * 32 + xc * 2;
+#pragma unroll
+    for(int k = 0; k < 10; k++) {
+      const bool ok = in && (k > 0 || xch > 0) && (k < 9 || xch < NCH - 1);
+      xv[k] = float2{0.f, 0.f};
+      if(ok) xv[k] = *(const float2 *)(sx + (k - 1) * 32);
+    }
+    const int fy = 2 * (y0 + zrow / TX) + (zph >> 1), fx = 2 * (x0 + zrow % TX) + (zph & 1);
+    const float *sz = dZ + ((b << (3 * LGD + 3)) + (size_t)(fy * Df + fx) * Df + zch * 16 + zh * 8) * COUT + c0 + zc * 2;
+#pragma unroll
+    for(int k = 0; k < 8; k++) zv[k] = *(const float2 *)(sz + k * COUT);
+  };
+  const int lane = tid & 63, w = tid >> 6, q = lane >> 4, n = lane & 15;
+  const int ay = w >> 2, ax = (w >> 1) & 1, h = w & 1;
+  cae_f32x4 acc[2][8] = {};
+  int task = blockIdx.x;
+  load(task);
+  while(task < ntask) {
+    __syncthreads();  // the previous tile's products are done with the chunks
+    if(xrow < HROWS) {
+#pragma unroll
+      for(int o = 0; o < 3; o++) {
+        cae_bf16x8 u, v;
+#pragma unroll
+        for(int k = 0; k < 8; k++) u[k] = (__bf16)xv[o + k].x, v[k] = (__bf16)xv[o + k].y;
+        char *d = xs + (((o * HROWS + xrow) * NCH + xch) * 32 + xc * 2) * 16;
+        *(cae_bf16x8 *)d = u, *(cae_bf16x8 *)(d + 16) = v;
+      }
+    }
+#pragma unroll
+    for(int az = 0; az < 2; az++) {
+      bf4 u, v;
+#pragma unroll
+      for(int k = 0; k < 4; k++) u[k] = (__bf16)zv[2 * k + az].x, v[k] = (__bf16)zv[2 * k + az].y;
+      char *d = zs + (((zrow * 8 + zph * 2 + az) * NCH + zch) * 16 + zc * 2) * 16 + zh * 8;
+      *(bf4 *)d = u, *(bf4 *)(d + 16) = v;
+    }
+    __syncthreads();
+    task += gridDim.x;
+    if(task < ntask) load(task);
+#pragma unroll
+    for(int ks = 0; ks < KS; ks++) {
+      // lane quarter q: chunk ks*4 + q of the tile
+      const int row = (ks * 4 + q) / NCH, ch = q % NCH, ly = row / TX, lx = row % TX;
+      cae_bf16x8 a[2];
+#pragma unroll
+      for(int az = 0; az < 2; az++)
+        a[az] = *(const cae_bf16x8 *)(zs + (((row * 8 + ay * 4 + ax * 2 + az) * NCH + ch) * 16 + n) * 16);
+#pragma unroll
+      for(int ty = 0; ty < 2; ty++)
+#pragma unroll
+        for(int tx = 0; tx < 2; tx++)
+#pragma unroll
+          for(int o = 0; o < 3; o++) {  // z offset o - 1: tap o - az of phase az
+            const int hr = (ly + ty + ay) * SX + lx + tx + ax;
+            const cae_bf16x8 v = *(const cae_bf16x8 *)(xs + (((o * HROWS + hr) * NCH + ch) * 32 + h * 16 + n) * 16);
+#pragma unroll
+            for(int az = 0; az < 2; az++) {
+              const int t = o - az;
+              if(t < 0 || t > 1) continue;
+              acc[az][(ty * 2 + tx) * 2 + t] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[az], v, acc[az][(ty * 2 + tx) * 2 + t], 0, 0, 0);
+            }
+          }
+    }
+  }
+  // part[slot][(a, t)][co][ci]
+  float *o = part + (size_t)blockIdx.x * (CAE_UPG / 16 * COUT);
+#pragma unroll
+  for(int az = 0; az < 2; az++)
+#pragma unroll
+    for(int t = 0; t < 8; t++)
+#pragma unroll
+      for(int r = 0; r < 4; r++)
+        o[(((ay * 4 + ax * 2 + az) * 8 + t) * COUT + c0 + q * 4 + r) * 32 + h * 16 + n] = acc[az][t][r];
+}
+
+// sum of nslot partial results of n values (n a multiple of 32) in a fixed order.  PITCH27: value i is
+// [i / 32][i % 32] of rows of 27 values in out.
+template<bool PITCH27>
+__global__ void __launch_bounds__(256) cae_wred_kernel(const float *__restrict__ part, int nslot, int n,
+                                                       float *__restrict__ out) {
+  __shared__ float s[256];
+  const int l = threadIdx.x & 31, g = threadIdx.x >> 5, i = blockIdx.x * 32 + l;
+  float v = 0.f;
+#pragma unroll 8
+  for(int k = g; k < nslot; k += 8) v += part[(size_t)k * n + i];
+  s[threadIdx.x] = v;
+  __syncthreads();
+  if(g) return;
+#pragma unroll
+  for(int k = 1; k < 8; k++) v += s[k * 32 + l];
+  if(!PITCH27) out[i] = v;
+  else if(l < 27) out[blockIdx.x * 27 + l] = v;
+}
+
+// dW[co][ci][tap] from G[(a, t)][co][ci]
+__global__ void cae_wup_sum_kernel(const float *__restrict__ G, int cout, float *__restrict__ dW) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if(i >= cout * 32 * 27) return;
+  const int tap = i % 27, c = i / 27, d[3] = {tap / 9, tap / 3 % 3, tap % 3};
+  float s = 0.f;
+#pragma unroll
+  for(int a = 0; a < 8; a++) {
+    int t = 0;
+    for(int k = 0; k < 3; k++) t = t * 2 + (d[k] > (a >> (2 - k) & 1));
+    s += G[(size_t)(a * 8 + t) * cout * 32 + c];
+  }
+  dW[i] = s;
+}
+
+// ---- weight gradients of the layers with one channel on one side ----------------------------------------
+//
+// 1 -> 16 (stride 2) and 16 -> 1: dW[m][tap] = sum_p V[p][m] S[.][tap] with V the 16-channel tensor on a grid of side
+// D and S the 1-channel tensor on the 32^3 grid, at 2p + d (STRIDE 2) or p - d (STRIDE 1).  M = 16 channels, N = 27
+// taps in two halves, K = positions.  V is read once, straight into the operand; S lies in LDS three times, at the
+// three z offsets, as runs of 8 positions.  A workgroup walks slabs of 4 planes.  `part` as above: [slot][16][32].
+// 64 blocks, below 45 us each (gathered per tap and padded to 32 channels: 541 us and 1450 us).
+template<int LGP, int STRIDE>
+__global__ void __launch_bounds__(256) cae_wgrad_vec_kernel(const float *__restrict__ V, const float *__restrict__ S,
+                                                            int ntask, float *__restrict__ part) {
+  constexpr int D = 1 << LGP, NCH = D / 8, TY = 4, SLABS = D / TY, RPK = 4 / NCH, W = 8 * STRIDE;
+  constexpr int SY = STRIDE * TY + 3 - STRIDE, SX = STRIDE * D + 3 - STRIDE, NR = SY * SX;
+  static_assert(STRIDE * D == 32, "S is on the 32^3 grid");
+  __shared__ __attribute__((aligned(16))) char ss[3 * NR * NCH * 16];
+  static_assert(sizeof(ss) >= 4 * 512 * 4, "holds the waves' sums");
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, n = lane & 15;
+  int toff[2];
+#pragma unroll
+  for(int h = 0; h < 2; h++) {
+    const int tap = min(h * 16 + n, 26), dy = tap / 9 - 1, dx = tap / 3 % 3 - 1, dz = tap % 3;
+    toff[h] = (dz * NR + (STRIDE == 1 ? (1 - dy) * SX + 1 - dx : (1 + dy) * SX + 1 + dx)) * NCH * 16;
+  }
+  cae_f32x4 acc[2] = {};
+  for(int task = blockIdx.x; task < ntask; task += gridDim.x) {
+    const size_t b = task / SLABS;
+    const int y0 = task % SLABS * TY;
+    const float *Sb = S + b * 32768;
+    __syncthreads();  // the previous slab's products are done with S
+    for(int e = threadIdx.x; e < NR * NCH; e += 256) {
+      const int ch = e % NCH, row = e / NCH, y = y0 * STRIDE + row / SX - 1, x = row % SX - 1;
+      float v[W + 2];  // cells ch*W - 1 ...
+#pragma unroll
+      for(int k = 0; k < W + 2; k++) v[k] = 0.f;
+      if((unsigned)y < 32u && (unsigned)x < 32u) {
+        const float *src = Sb + (y * 32 + x) * 32 + ch * W;
+#pragma unroll
+        for(int k = 0; k < W; k += 4) {
+          const float4 f = *(const float4 *)(src + k);
+          v[k + 1] = f.x, v[k + 2] = f.y, v[k + 3] = f.z, v[k + 4] = f.w;
+        }
+        if(ch > 0) v[0] = src[-1];
+        if(ch < NCH - 1) v[W + 1] = src[W];
+      }
+#pragma unroll
+      for(int o = 0; o < 3; o++) {
+        cae_bf16x8 u;
+#pragma unroll
+        for(int k = 0; k < 8; k++) u[k] = (__bf16)v[STRIDE == 1 ? k + 2 - o : 2 * k + o];
+        *(cae_bf16x8 *)(ss + ((o * NR + row) * NCH + ch) * 16) = u;
+      }
+    }
+    __syncthreads();
+    const float *Vb = V + ((b << (3 * LGP)) + ((size_t)y0 << (2 * LGP))) * 16;
+#pragma unroll 4
+    for(int k = w; k < TY * D / RPK; k += 4) {
+      const int row = k * RPK + q / NCH, ch = q % NCH, ly = row >> LGP, x = row & (D - 1);
+      const float *src = Vb + ((row << LGP) + ch * 8) * 16 + n;
+      cae_bf16x8 a;
+#pragma unroll
+      for(int t = 0; t < 8; t++) a[t] = (__bf16)src[t * 16];
+      const char *base = ss + ((STRIDE * ly * SX + STRIDE * x) * NCH + ch) * 16;
+#pragma unroll
+      for(int h = 0; h < 2; h++)
+        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, *(const cae_bf16x8 *)(base + toff[h]), acc[h], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+  float *red = (float *)ss;
+#pragma unroll
+  for(int h = 0; h < 2; h++)
+#pragma unroll
+    for(int r = 0; r < 4; r++) red[w * 512 + (q * 4 + r) * 32 + h * 16 + n] = acc[h][r];
+  __syncthreads();
+  for(int i = threadIdx.x; i < 512; i += 256)
+    part[(size_t)blockIdx.x * 512 + i] = red[i] + red[512 + i] + red[1024 + i] + red[1536 + i];
+}
+
 // dW[co][ci][tap] += sum_{b, p} dZ[b][p][co] * X[b][q(p, tap)][ci] over a chunk of CAE_WG_CHUNK positions of
 // one block: M = output channels, N = 32 (tap, ci) pairs n = tap*CIN + ci, K = positions.  Long chunks keep
 // the atomic additions of the partial sums few (they all land on the layer's small dW).
@@ -622,6 +842,9 @@ __global__ void cae_scatter_kernel(const float *__restrict__ rec, const CaeBlock
 
 // ---- host side -------------------------------------------------------------------------------------
 
+// partial weight gradients: 256 workgroups of an upsampling layer (one per CU)
+constexpr int CAE_PART = 256 * CAE_UPG;
+
 static int lg2(int d) {
   int l = 0;
   while((1 << l) < d) l++;
@@ -633,7 +856,7 @@ static int fwd_ksteps(int l) { return kKind[l] == K_UP || l == CAE_LAYERS - 1 ? 
 
 CaeWork::~CaeWork() {
   for(int l = 0; l < CAE_LAYERS; l++) (void)hipFree(z[l]), (void)hipFree(a[l]);
-  for(void *p : {(void *)g0, (void *)g1, (void *)g2, (void *)x, (void *)scale, (void *)ss, (void *)part, org})
+  for(void *p : {(void *)g0, (void *)g1, (void *)g2, (void *)x, (void *)scale, (void *)ss, (void *)part, (void *)wpart, org})
     (void)hipFree(p);
 }
 
@@ -721,7 +944,7 @@ int cae_reserve(CaeWork &w, int nb, bool train) {
     (void)hipFree(w.z[l]), (void)hipFree(w.a[l]);
     w.z[l] = w.a[l] = nullptr;
   }
-  for(float **p : {&w.g0, &w.g1, &w.g2, &w.x, &w.scale, &w.ss, &w.part}) (void)hipFree(*p), *p = nullptr;
+  for(float **p : {&w.g0, &w.g1, &w.g2, &w.x, &w.scale, &w.ss, &w.part, &w.wpart}) (void)hipFree(*p), *p = nullptr;
   (void)hipFree(w.org);
   w.org = nullptr;
   w.cap = 0, w.train = false;
@@ -746,6 +969,7 @@ int cae_reserve(CaeWork &w, int nb, bool train) {
     KL_HIP(hipMalloc(&w.g0, gmax * 4));
     KL_HIP(hipMalloc(&w.g1, gmax * 4));
     KL_HIP(hipMalloc(&w.g2, umax * 4));
+    KL_HIP(hipMalloc(&w.wpart, ((size_t)CAE_PART + CAE_UPG * 2) * 4));
   }
   w.cap = nb, w.train = train;
   return KLRTM_OK;
@@ -831,29 +1055,54 @@ static int layer_dgrad(const ConvAE &c, const CaeWork &w, int l, const float *dz
   return check_launch("cae_conv_kernel");
 }
 
-// weight and bias gradients of layer l (added to d_grad) from its input and its pre-activation gradient
-static int layer_wgrad(ConvAE &c, int l, const float *in, const float *dz, int nb) {
+// weight and bias gradients of layer l into d_grad (cleared before) from its input and its pre-activation gradient
+static int layer_wgrad(ConvAE &c, CaeWork &w, int l, const float *in, const float *dz, int nb) {
   const int lgo = lg2(kDout[l]), lgg = lg2(kDin[l]);
   const long P = 1L << (3 * lgo);
-  const int ntile = (kCin[l] * 27 + 31) / 32;
-  const dim3 grid((unsigned)((ntile + 3) / 4), (unsigned)((P + CAE_WG_CHUNK - 1) / CAE_WG_CHUNK), (unsigned)nb);
   float *dW = c.d_grad + c.w_off[l];
-  const int mode = kKind[l] == K_DOWN ? G_DOWN : kKind[l] == K_UP ? G_UP : G_SAME;
-#define CAE_W(CI, M) \
-  hipLaunchKernelGGL((cae_wgrad_kernel<CI, M>), grid, dim3(256), 0, stream(), in, dz, kCout[l], lgo, lgg, dW)
-  switch(kCin[l] * 8 + mode) {
-  case 1 * 8 + G_DOWN: CAE_W(1, G_DOWN); break;
-  case 16 * 8 + G_DOWN: CAE_W(16, G_DOWN); break;
-  case 32 * 8 + G_SAME: CAE_W(32, G_SAME); break;
-  case 4 * 8 + G_SAME: CAE_W(4, G_SAME); break;
-  case 32 * 8 + G_UP: CAE_W(32, G_UP); break;
-  case 16 * 8 + G_SAME: CAE_W(16, G_SAME); break;
-  default: set_error("autoencoder layer %d has no weight-gradient kernel", l); return KLRTM_EINVAL;
-  }
-#undef CAE_W
   const long n = (long)nb * P * kCout[l];
   hipLaunchKernelGGL(cae_bgrad_kernel, dim3((unsigned)((n + 8191) / 8192)), dim3(256), 0, stream(), dz, n, kCout[l],
                      c.d_grad + c.b_off[l]);
+  if(kKind[l] == K_UP) {
+    const int ng = CAE_UPG / 16 * kCout[l], tiles = kDin[l] == 8 ? 8 : 64, ntask = nb * tiles;
+    const int slots = std::min(ntask, CAE_PART / ng);
+    const dim3 grid((unsigned)slots, (unsigned)(kCout[l] / 16));
+    float *G = w.wpart + CAE_PART;
+    if(kCout[l] == 32 && kDin[l] == 8)
+      hipLaunchKernelGGL((cae_wgrad_up_kernel<32, 3>), grid, dim3(512), 0, stream(), in, dz, ntask, w.wpart);
+    else if(kCout[l] == 16 && kDin[l] == 16)
+      hipLaunchKernelGGL((cae_wgrad_up_kernel<16, 4>), grid, dim3(512), 0, stream(), in, dz, ntask, w.wpart);
+    else {
+      set_error("autoencoder layer %d has no weight-gradient kernel", l);
+      return KLRTM_EINVAL;
+    }
+    hipLaunchKernelGGL(cae_wred_kernel<false>, dim3((unsigned)(ng / 32)), dim3(256), 0, stream(), w.wpart, slots, ng, G);
+    hipLaunchKernelGGL(cae_wup_sum_kernel, dim3((unsigned)((kCout[l] * 32 * 27 + 255) / 256)), dim3(256), 0, stream(), G,
+                       kCout[l], dW);
+    return check_launch("cae_wgrad_up_kernel");
+  }
+  if(kCin[l] == 1 || kCout[l] == 1) {
+    const bool first = kCin[l] == 1;
+    const int ntask = nb * (first ? 4 : 8), slots = std::min(ntask, 1024);
+    if(first)
+      hipLaunchKernelGGL((cae_wgrad_vec_kernel<4, 2>), dim3((unsigned)slots), dim3(256), 0, stream(), dz, in, ntask, w.wpart);
+    else
+      hipLaunchKernelGGL((cae_wgrad_vec_kernel<5, 1>), dim3((unsigned)slots), dim3(256), 0, stream(), in, dz, ntask, w.wpart);
+    hipLaunchKernelGGL(cae_wred_kernel<true>, dim3(16), dim3(256), 0, stream(), w.wpart, slots, 512, dW);
+    return check_launch("cae_wgrad_vec_kernel");
+  }
+  const int ntile = (kCin[l] * 27 + 31) / 32;
+  const dim3 grid((unsigned)((ntile + 3) / 4), (unsigned)((P + CAE_WG_CHUNK - 1) / CAE_WG_CHUNK), (unsigned)nb);
+  const int mode = kKind[l] == K_DOWN ? G_DOWN : G_SAME;
+#define CAE_W(CI, M) \
+  hipLaunchKernelGGL((cae_wgrad_kernel<CI, M>), grid, dim3(256), 0, stream(), in, dz, kCout[l], lgo, lgg, dW)
+  switch(kCin[l] * 8 + mode) {
+  case 16 * 8 + G_DOWN: CAE_W(16, G_DOWN); break;
+  case 32 * 8 + G_SAME: CAE_W(32, G_SAME); break;
+  case 4 * 8 + G_SAME: CAE_W(4, G_SAME); break;
+  default: set_error("autoencoder layer %d has no weight-gradient kernel", l); return KLRTM_EINVAL;
+  }
+#undef CAE_W
   return check_launch("cae_wgrad_kernel");
 }
 
@@ -881,7 +1130,7 @@ int cae_loss_grad(ConvAE &c, const float *x, int nb) {
   float *dz = w.g0, *din = w.g1;
   for(int l = CAE_LAYERS - 1; l >= 0; l--) {
     const float *in = l == 0 ? x : w.a[l - 1];
-    if((rc = layer_wgrad(c, l, in, dz, nb))) return rc;
+    if((rc = layer_wgrad(c, w, l, in, dz, nb))) return rc;
     if(l == 0) break;
     if((rc = layer_dgrad(c, w, l, dz, din, w.g2, nb))) return rc;
     std::swap(dz, din);
