@@ -55,6 +55,14 @@ struct CfdPassArgs {
 // the segment, results of clamped loads discarded), and PML state outside a
 // layer is reached through a buffer resource whose out-of-range accesses the
 // hardware drops.
+//
+// A small grid has fewer waves than SIMDs (229 for 121^3), so a line costs its
+// serial chain.  Whole batches are straight code: no check per sample, running
+// addresses, and the batch's plan rows read together before the prefetch.  With
+// a check and a scalar load per row a sample of the two sweeps took 1700 cycles
+// (y gradient of 121^3: 87 us), now 1200 (61 us); 31 + 35 instructions of a row
+// are about 300 of them, the rest waits on memory (of lines and of code: twice
+// the prefetch depth gained nothing).  On 400^3 (2500 waves): 689 -> 655 us.
 
 // PML slot of one damped derivative component along the sweep: the state of
 // sample ii sits at byte offset off + ii*step (both per lane) of the resource spanning both
@@ -99,14 +107,14 @@ __device__ __forceinline__ void cross_setup(const PmlDesc &P, int round, int ax,
 
 template<int AXIS, int PASS, int MODEL>
 struct LineSweep {
-  // streams of the backward sweep
-  const float *t;  // b' (the forward sweep's output line)
+  // streams of the backward sweep (tmp holds b', the forward sweep's output)
   float *tmp, *pr, *pz, *pb;
   const float *vel, *w1, *eps, *del, *pjx, *pjy;
   const float *prl, *pjyl;  // pr, pjy for loads (another valid stream in 2D, where the value is unused)
   bool jzl;                 // IRREGULAR z grid: the Dz term of P_DIV3_STEP takes this lane's jacobz
   float jzv;
-  size_t base, s;
+  size_t base;
+  uint32_t s;  // cells between samples of the line
   const cfloat *U;
   int n, ny;
   float Y0, Y1, Y2, Y3;
@@ -121,6 +129,9 @@ struct LineSweep {
                            : PASS == P_GRAD_SCALAR ? (MODEL == KLRTM_ISO ? 0 : MODEL == KLRTM_VTI ? 4 : 6)
                            : PASS == P_DIV ? 2 : PASS == P_DIV_STEP ? 3 : 5;
 
+  // cell offset of sample ii: one 32 x 32 -> 64 bit product
+  __device__ __forceinline__ size_t row(int ii) const { return (uint64_t)(uint32_t)ii * s; }
+
   template<bool OWN, bool CROSS, int NB>
   struct Batch {
     float tv[NB], o[E > 0 ? E : 1][NB], qo[OWN ? NB : 1], q1[CROSS ? NB : 1], q2[CROSS ? NB : 1];
@@ -128,11 +139,12 @@ struct LineSweep {
 
   template<bool OWN, bool CROSS, int NB>
   __device__ __forceinline__ void load(Batch<OWN, CROSS, NB> &B, int hi, int lo) {
+    uint32_t o1 = CROSS ? cs1.off + (uint32_t)hi * cs1.step : 0, o2 = CROSS ? cs2.off + (uint32_t)hi * cs2.step : 0;
+    size_t c = base + row(max(hi, lo));
+    const float *qp = OWN ? qo + (size_t)(max(hi, lo) - jbase) * qo_js : nullptr;
 #pragma unroll
     for(int j = 0; j < NB; j++) {
-      const int ii = max(hi - j, lo);
-      const size_t c = base + (size_t)ii * s;
-      B.tv[j] = t[(size_t)ii * s];
+      B.tv[j] = tmp[c];
       if(PASS == P_GRAD_SCALAR && MODEL != KLRTM_ISO) {
         B.o[0][j] = prl[c], B.o[1][j] = pz[c], B.o[2][j] = eps[c], B.o[3][j] = del[c];
         if(MODEL == KLRTM_TTI) B.o[4][j] = pjx[c], B.o[5][j] = pjyl[c];
@@ -142,24 +154,26 @@ struct LineSweep {
       } else if(PASS == P_DIV3_STEP) {  // pr carries Dx here, pz Dz
         B.o[0][j] = pb[c], B.o[1][j] = vel[c], B.o[2][j] = pr[c], B.o[3][j] = pz[c], B.o[4][j] = w1[c];
       }
-      if(OWN) B.qo[j] = qo[(size_t)(ii - jbase) * qo_js];
+      if(OWN) B.qo[j] = *qp, qp -= hi - j > lo ? qo_js : 0;
       if(CROSS) {
-        B.q1[j] = buf_ld(cs1.rs, cs1.off + (uint32_t)ii * cs1.step, 0);
-        B.q2[j] = buf_ld(cs2.rs, cs2.off + (uint32_t)ii * cs2.step, 0);
+        // (rows below lo: the value is not used, and the resource bounds the access)
+        B.q1[j] = buf_ld(cs1.rs, o1, 0), o1 -= cs1.step;
+        B.q2[j] = buf_ld(cs2.rs, o2, 0), o2 -= cs2.step;
       }
+      c -= hi - j > lo ? (size_t)s : 0;
     }
   }
 
-  // back substitution of sample ii (rows ii >= n-4 use only the solved neighbours that exist)
-  __device__ __forceinline__ float solve(int ii, float v, bool edge) {
+  // back substitution of sample ii (rows ii >= n-4, `edge`, use only the solved neighbours that exist)
+  __device__ __forceinline__ float solve(int ii, const float (&u)[5], float v, bool edge) {
     if(edge) {
       const int l = n - 1 - ii;
-      if(l >= 1) v = v - U[ii * 5 + 1] * Y0;
-      if(l >= 2) v = v - U[ii * 5 + 2] * Y1;
-      if(l >= 3) v = v - U[ii * 5 + 3] * Y2;
-      v = v / U[ii * 5];
+      if(l >= 1) v = v - u[1] * Y0;
+      if(l >= 2) v = v - u[2] * Y1;
+      if(l >= 3) v = v - u[3] * Y2;
+      v = v / u[0];
     } else {
-      v = (v - U[ii * 5 + 1] * Y0 - U[ii * 5 + 2] * Y1 - U[ii * 5 + 3] * Y2 - U[ii * 5 + 4] * Y3) / U[ii * 5];
+      v = (v - u[1] * Y0 - u[2] * Y1 - u[3] * Y2 - u[4] * Y3) / u[0];
     }
     Y3 = Y2, Y2 = Y1, Y1 = Y0, Y0 = v;
     return v;
@@ -167,10 +181,10 @@ struct LineSweep {
 
   // PML rounds (bgprtm/PML.cpp:62-70) of the own axis then the cross axes, and the pass epilogue
   template<bool OWN, bool CROSS, int NB>
-  __device__ __forceinline__ void finish(const Batch<OWN, CROSS, NB> &B, int j, int ii, float v) {
+  __device__ __forceinline__ void finish(const Batch<OWN, CROSS, NB> &B, int j, int ii, size_t c, uint32_t o1, uint32_t o2,
+                                         float gg, float v) {
     float g = v;
     if(OWN) {
-      const float gg = go[ii - jbase];
       float qi = (1.0f - gg) / (1.0f + gg) * B.qo[j] - gg * 2.0f / (1.0f - gg * gg) * g;
       qo[(size_t)(ii - jbase) * qo_js] = qi;
       g = qi + g / (1.0f - gg);
@@ -179,13 +193,12 @@ struct LineSweep {
       float qi = cs1.a * B.q1[j] - cs1.b * g;
       float r = qi + g / cs1.d;
       g = cs1.on ? r : g;
-      buf_st(qi, cs1.rs, cs1.off + (uint32_t)ii * cs1.step, 0);
+      buf_st(qi, cs1.rs, o1, 0);
       qi = cs2.a * B.q2[j] - cs2.b * g;
       r = qi + g / cs2.d;
       g = cs2.on ? r : g;
-      buf_st(qi, cs2.rs, cs2.off + (uint32_t)ii * cs2.step, 0);
+      buf_st(qi, cs2.rs, o2, 0);
     }
-    const size_t c = base + (size_t)ii * s;
     if(PASS == P_GRAD) {
       tmp[c] = g;
     } else if(PASS == P_GRAD_SCALAR && MODEL == KLRTM_ISO) {
@@ -211,25 +224,59 @@ struct LineSweep {
     }
   }
 
-  // samples ii, ii-1, ... of batch B (cnt of them); the edge rows take the short back substitution
-  template<bool OWN, bool CROSS, int NB>
-  __device__ __forceinline__ void compute(const Batch<OWN, CROSS, NB> &B, int ii, int cnt) {
+  // samples ii, ii-1, ... of batch B with their plan rows u and layer profile gg.  CHECK: cnt of them (rows read as they are needed), and
+  // the edge rows take the short back substitution; otherwise the batch lies below the edge rows
+  template<bool CHECK, bool OWN, bool CROSS, int NB>
+  __device__ __forceinline__ void compute(const Batch<OWN, CROSS, NB> &B, const float (&u)[CHECK ? 1 : NB][5],
+                                          const float (&gg)[CHECK ? 1 : NB], int ii, int cnt) {
+    uint32_t o1 = CROSS ? cs1.off + (uint32_t)ii * cs1.step : 0, o2 = CROSS ? cs2.off + (uint32_t)ii * cs2.step : 0;
+    size_t c = base + row(ii);
 #pragma unroll
-    for(int j = 0; j < NB; j++)
-      if(j < cnt) finish<OWN, CROSS, NB>(B, j, ii - j, solve(ii - j, B.tv[j], ii - j >= n - 4));
+    for(int j = 0; j < NB; j++) {
+      if(CHECK) {
+        if(j < cnt) {
+          float r[5];
+#pragma unroll
+          for(int k = 0; k < 5; k++) r[k] = U[(ii - j) * 5 + k];
+          finish<OWN, CROSS, NB>(B, j, ii - j, c, o1, o2, OWN ? go[ii - j - jbase] : 0.f,
+                                 solve(ii - j, r, B.tv[j], ii - j >= n - 4));
+        }
+      } else {
+        finish<OWN, CROSS, NB>(B, j, ii - j, c, o1, o2, gg[j], solve(ii - j, u[j], B.tv[j], false));
+      }
+      c -= s;
+      if(CROSS) o1 -= cs1.step, o2 -= cs2.step;
+    }
   }
-  // one batch: prefetch the next into nxt (unless cur is the last), then solve cur
+  // one batch: prefetch the next into nxt (clamped to the segment: past its end the loads repeat), then solve cur.
+  // The plan rows of a whole batch are asked for before the prefetch and pinned after it, a few wide scalar loads
+  // with one wait; left to itself the compiler loads each row where it is used and waits for it there.
   template<bool OWN, bool CROSS, int NB>
   __device__ __forceinline__ bool half(const Batch<OWN, CROSS, NB> &cur, Batch<OWN, CROSS, NB> &nxt, int &ii, int lo) {
     const int left = ii - lo + 1;
-    if(left <= NB) {
-      compute<OWN, CROSS, NB>(cur, ii, left);
-      return false;
+    if(left < NB || ii >= n - 4) {
+      const float none[1][5] = {}, nog[1] = {};
+      load<OWN, CROSS, NB>(nxt, ii - NB, lo);
+      compute<true, OWN, CROSS, NB>(cur, none, nog, ii, left);
+    } else {
+      float u[NB][5], gg[NB];
+      const cfloat *up = U + (size_t)(ii - NB + 1) * 5, *gp = OWN ? go + (ii - NB + 1 - jbase) : up;
+#pragma unroll
+      for(int j = 0; j < NB; j++) {
+#pragma unroll
+        for(int k = 0; k < 5; k++) u[j][k] = up[(NB - 1 - j) * 5 + k];
+        gg[j] = OWN ? gp[NB - 1 - j] : 0.f;
+      }
+      load<OWN, CROSS, NB>(nxt, ii - NB, lo);
+#pragma unroll
+      for(int j = 0; j < NB; j++) {
+        asm volatile("" : "+s"(u[j][0]), "+s"(u[j][1]), "+s"(u[j][2]), "+s"(u[j][3]), "+s"(u[j][4]));
+        if(OWN) asm volatile("" : "+s"(gg[j]));
+      }
+      compute<false, OWN, CROSS, NB>(cur, u, gg, ii, NB);
     }
-    load<OWN, CROSS, NB>(nxt, ii - NB, lo);
-    compute<OWN, CROSS, NB>(cur, ii, NB);
     ii -= NB;
-    return true;
+    return left > NB;
   }
 
   // samples hi down to lo; batches alternate between two register sets so a
@@ -237,7 +284,7 @@ struct LineSweep {
   template<bool OWN, bool CROSS>
   __device__ __forceinline__ void segment(int hi, int lo) {
     constexpr int streams = 1 + E + (OWN ? 1 : 0) + (CROSS ? 2 : 0);
-    constexpr int NB = streams >= 8 ? 4 : streams >= 5 ? 6 : streams >= 3 ? 8 : 12;
+    constexpr int NB = streams >= 8 ? 4 : streams >= 5 ? 6 : 8;
     Batch<OWN, CROSS, NB> b0, b1;
     int ii = hi;
     load<OWN, CROSS, NB>(b0, ii, lo);
@@ -260,9 +307,10 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
   const size_t nxz = (size_t)nx * nz;
   int cx = 0, cy = 0, n;
   const int cz = (int)(b % nz);
-  size_t base, s;
-  if(AXIS == AXX) cy = (int)(b / nz), base = (size_t)cy * nxz + cz, s = (size_t)nz, n = nx;
-  else cx = (int)(b / nz), base = (size_t)cx * nz + cz, s = nxz, n = ny;
+  size_t base;
+  uint32_t s;
+  if(AXIS == AXX) cy = (int)(b / nz), base = (size_t)cy * nxz + cz, s = (uint32_t)nz, n = nx;
+  else cx = (int)(b / nz), base = (size_t)cx * nz + cz, s = (uint32_t)nxz, n = ny;
   const cfloat *A = as_const(a.am);
   const cfloat *Lw = as_const(a.bl);
   const float *x = in + base;
@@ -271,7 +319,7 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
   // ---- forward sweep: RHS band multiply + elimination (bgprtm/FdEngine_cfd.cpp:170-230)
   // window sample k, zero beyond the line; the load itself is always issued (clamped)
   auto xload = [&](int k) {
-    const float v = x[(size_t)min(k, n - 1) * s];
+    const float v = x[(uint64_t)(uint32_t)min(k, n - 1) * s];
     return k < n ? v : 0.f;
   };
   constexpr int NF = 12;  // interior rows per batch
@@ -291,7 +339,7 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
     for(int k = 0; k < 10; k++) X[k] = X[k + 1];
     X[10] = v;
   };
-  auto eliminate = [&](int i, float acc) {
+  auto eliminate = [&](int i, float acc) __attribute__((always_inline)) {  // (i >= 5: all four terms)
     if(i >= 4) acc = acc - Lw[(i - 4) * 4 + 3] * B3;
     if(i >= 3) acc = acc - Lw[(i - 3) * 4 + 2] * B2;
     if(i >= 2) acc = acc - Lw[(i - 2) * 4 + 1] * B1;
@@ -311,28 +359,55 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
   auto interior = [&]() {
     return a55 * (X[6] - X[4]) + a56 * (X[7] - X[3]) + a57 * (X[8] - X[2]) + a58 * (X[9] - X[1]) + a59 * (X[10] - X[0]);
   };
-  // interior rows [i, n-5): cur holds window samples i+6.., the next batch is prefetched into nxt
+  auto eliminate4 = [&](int i, float acc) __attribute__((always_inline)) {
+    acc = acc - Lw[(i - 4) * 4 + 3] * B3;
+    acc = acc - Lw[(i - 3) * 4 + 2] * B2;
+    acc = acc - Lw[(i - 2) * 4 + 1] * B1;
+    acc = acc - Lw[(i - 1) * 4 + 0] * B0;
+    B3 = B2, B2 = B1, B1 = B0, B0 = acc;
+    return acc;
+  };
+  // interior rows [i, n-5): cur holds window samples i+6.., the next batch is prefetched into nxt.  While that lies
+  // within the line nothing is checked, and the batch's elimination rows are asked for before the prefetch and
+  // pinned after it (see LineSweep::half).
   auto fhalf = [&](const float(&cur)[NF], float(&nxt)[NF], int &i) __attribute__((always_inline)) {
     const int left = (n - 5) - i;
-    if(left <= NF) {
+    float *o = t + (uint64_t)(uint32_t)i * s;
+    if(i + 2 * NF + 6 <= n) {
+      float lw[NF][4];
+      const cfloat *lp = Lw + (size_t)(i - 4) * 4;
+#pragma unroll
+      for(int j = 0; j < NF; j++)
+#pragma unroll
+        for(int k = 0; k < 4; k++) lw[j][k] = lp[(j + 3 - k) * 4 + k];
+      const float *src = x + (uint64_t)(uint32_t)(i + NF + 6) * s;
+#pragma unroll
+      for(int j = 0; j < NF; j++) nxt[j] = *src, src += s;
+#pragma unroll
+      for(int j = 0; j < NF; j++) asm volatile("" : "+s"(lw[j][0]), "+s"(lw[j][1]), "+s"(lw[j][2]), "+s"(lw[j][3]));
+#pragma unroll
+      for(int j = 0; j < NF; j++) {
+        float acc = interior();
+        acc = acc - lw[j][3] * B3;
+        acc = acc - lw[j][2] * B2;
+        acc = acc - lw[j][1] * B1;
+        acc = acc - lw[j][0] * B0;
+        B3 = B2, B2 = B1, B1 = B0, B0 = acc;
+        *o = acc, o += s;
+        shift_in(cur[j]);
+      }
+    } else {
+#pragma unroll
+      for(int j = 0; j < NF; j++) nxt[j] = xload(i + NF + 6 + j);
 #pragma unroll
       for(int j = 0; j < NF; j++)
         if(j < left) {
-          t[(size_t)(i + j) * s] = eliminate(i + j, interior());
+          *o = eliminate4(i + j, interior()), o += s;
           shift_in(cur[j]);
         }
-      i += left;
-      return false;
-    }
-#pragma unroll
-    for(int j = 0; j < NF; j++) nxt[j] = xload(i + NF + 6 + j);
-#pragma unroll
-    for(int j = 0; j < NF; j++) {
-      t[(size_t)(i + j) * s] = eliminate(i + j, interior());
-      shift_in(cur[j]);
     }
     i += NF;
-    return true;
+    return left > NF;
   };
   {
     int i = 5;
@@ -345,13 +420,13 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
     float acc = 0.f;
 #pragma unroll
     for(int j = 0; j < 10 - r; j++) acc = acc - A[54 - r - 5 * j] * X[j];
-    t[(size_t)ii * s] = eliminate(ii, acc);
+    t[(uint64_t)(uint32_t)ii * s] = eliminate4(ii, acc);
     if(r < 4) shift_in(0.f);  // samples n+1.. lie beyond the line
   }
 
   // ---- backward sweep + epilogue (bgprtm/FdEngine_cfd.cpp:231-254), by PML segment
   LineSweep<AXIS, PASS, MODEL> L;
-  L.t = t, L.tmp = tmp, L.pr = pr, L.pz = pz, L.pb = pb;
+  L.tmp = tmp, L.pr = pr, L.pz = pz, L.pb = pb;
   L.vel = vel, L.w1 = w1, L.eps = eps, L.del = del, L.pjx = pjx, L.pjy = pjy;
   L.prl = ny > 1 ? pr : pz, L.pjyl = ny > 1 ? pjy : pjx;
   L.base = base, L.s = s, L.U = as_const(a.bm), L.n = n, L.ny = ny;
@@ -411,14 +486,16 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
 // (backward) in place, and both go back to global memory through the same
 // transposed tiles, so every global access of the pass is coalesced.
 // Interior chunks are fully unrolled: the 11-sample window lives in renamed
-// registers and the plan rows of a chunk arrive as a few scalar loads.
+// registers and the plan rows and samples of half a chunk are read before its
+// solves (121^3: 76 -> 70 us).
 // Global memory is reached through per-wave buffer resources; tile elements
 // beyond the line or the last line get an out-of-range offset, so their loads
 // return 0 and their stores are dropped, and no access needs a branch.
 // Per-sample arithmetic is identical to cfd_line_kernel.
 constexpr int ZC = 16, ZSP = ZC + 1;  // chunk length, LDS row pitch (odd: conflict-free)
 constexpr int ZLPR = 64 / ZC;         // lines per tile row
-constexpr int ZU = 8;                 // samples per unrolled step of an interior chunk sweep
+constexpr int ZU = 8;                 // samples per unrolled step of an interior chunk sweep (half a chunk)
+static_assert(ZC == 2 * ZU, "a step's window samples lie in one or two chunks");
 
 struct ZCross {  // cross-axis PML slot of one line: state offset of z = 0 (OOR: outside), coefficients
   uint32_t off;
@@ -544,21 +621,32 @@ __global__ void __launch_bounds__(64) cfd_zline_kernel(const float *in, float *t
       // sit in the two staged chunks (zero beyond the line)
 #pragma unroll 1
       for(int jb = 0; jb < ZC; jb += ZU) {
+        // the step's window samples and elimination rows first: one wait instead of one a row
+        float xw[ZU], lw[ZU][4];
+        const cfloat *lp = Lw + (size_t)(i0 + jb - 4) * 4;
+        const float *c1 = cur + jb + 6, *c2 = jb + ZU < ZC ? c1 : nxt + jb + 6 - ZC;
+#pragma unroll
+        for(int jj = 0; jj < ZU; jj++) xw[jj] = jj + 6 < ZU ? c1[jj] : c2[jj];
+#pragma unroll
+        for(int jj = 0; jj < ZU; jj++)
+#pragma unroll
+          for(int k = 0; k < 4; k++) lw[jj][k] = lp[(jj + 3 - k) * 4 + k];
+#pragma unroll
+        for(int jj = 0; jj < ZU; jj++)
+          asm volatile("" : "+s"(lw[jj][0]), "+s"(lw[jj][1]), "+s"(lw[jj][2]), "+s"(lw[jj][3]), "+v"(xw[jj]));
 #pragma unroll
         for(int jj = 0; jj < ZU; jj++) {
-          const int j = jb + jj, i = i0 + j;
           float acc = a55 * (X[6] - X[4]) + a56 * (X[7] - X[3]) + a57 * (X[8] - X[2]) + a58 * (X[9] - X[1]) +
                       a59 * (X[10] - X[0]);
-          acc = acc - Lw[(i - 4) * 4 + 3] * B3;
-          acc = acc - Lw[(i - 3) * 4 + 2] * B2;
-          acc = acc - Lw[(i - 2) * 4 + 1] * B1;
-          acc = acc - Lw[(i - 1) * 4 + 0] * B0;
+          acc = acc - lw[jj][3] * B3;
+          acc = acc - lw[jj][2] * B2;
+          acc = acc - lw[jj][1] * B1;
+          acc = acc - lw[jj][0] * B0;
           B3 = B2, B2 = B1, B1 = B0, B0 = acc;
-          const float xn = j + 6 < ZC ? cur[j + 6] : nxt[j + 6 - ZC];
-          cur[j] = acc;
+          cur[jb + jj] = acc;
 #pragma unroll
           for(int k = 0; k < 10; k++) X[k] = X[k + 1];
-          X[10] = xn;
+          X[10] = xw[jj];
         }
       }
     } else {
@@ -710,11 +798,21 @@ __global__ void __launch_bounds__(64) cfd_zline_kernel(const float *in, float *t
       // full chunk (only the last chunk can be short, and it holds the edge rows)
 #pragma unroll 1
       for(int jb = ZC - ZU; jb >= 0; jb -= ZU) {
+        float rv[ZU], u[ZU][5];
+        const cfloat *up = U + (size_t)(i0 + jb) * 5;
+#pragma unroll
+        for(int jj = 0; jj < ZU; jj++) {
+          rv[jj] = row[jb + jj];
+#pragma unroll
+          for(int k = 0; k < 5; k++) u[jj][k] = up[jj * 5 + k];
+        }
+#pragma unroll
+        for(int jj = 0; jj < ZU; jj++)
+          asm volatile("" : "+s"(u[jj][0]), "+s"(u[jj][1]), "+s"(u[jj][2]), "+s"(u[jj][3]), "+s"(u[jj][4]), "+v"(rv[jj]));
 #pragma unroll
         for(int jj = ZU - 1; jj >= 0; jj--) {
-          const int j = jb + jj, i = i0 + j;
-          float v = (row[j] - U[i * 5 + 1] * Y0 - U[i * 5 + 2] * Y1 - U[i * 5 + 3] * Y2 - U[i * 5 + 4] * Y3) / U[i * 5];
-          row[j] = v;
+          float v = (rv[jj] - u[jj][1] * Y0 - u[jj][2] * Y1 - u[jj][3] * Y2 - u[jj][4] * Y3) / u[jj][0];
+          row[jb + jj] = v;
           Y3 = Y2, Y2 = Y1, Y1 = Y0, Y0 = v;
         }
       }
