@@ -503,6 +503,8 @@ __global__ void cae_wup_sum_kernel(const float *__restrict__ G, int cout, float 
 // taps in two halves, K = positions.  V is read once, straight into the operand; S lies in LDS three times, at the
 // three z offsets, as runs of 8 positions.  A workgroup walks slabs of 4 planes.  `part` as above: [slot][16][32].
 // 64 blocks, below 45 us each (gathered per tap and padded to 32 channels: 541 us and 1450 us).
+// (S may be the caller's tensor, aligned to its elements only: the hardware's wide loads accept that)
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 template<int LGP, int STRIDE>
 __global__ void __launch_bounds__(256) cae_wgrad_vec_kernel(const float *__restrict__ V, const float *__restrict__ S,
                                                             int ntask, float *__restrict__ part) {
@@ -533,7 +535,7 @@ __global__ void __launch_bounds__(256) cae_wgrad_vec_kernel(const float *__restr
         const float *src = Sb + (y * 32 + x) * 32 + ch * W;
 #pragma unroll
         for(int k = 0; k < W; k += 4) {
-          const float4 f = *(const float4 *)(src + k);
+          const f4u f = *(const f4u *)(src + k);
           v[k + 1] = f.x, v[k + 2] = f.y, v[k + 3] = f.z, v[k + 4] = f.w;
         }
         if(ch > 0) v[0] = src[-1];

@@ -80,3 +80,21 @@ def test_weight_gradient_of_every_tap(klrtm, nb):
         print(f"[convae] layer {l}: largest tap error {max(e):.2e}", flush=True)
         worst = max(worst, max(e))
     assert worst < 5e-2
+
+
+def test_gradient_of_a_shifted_input(klrtm):
+    """A batch that starts one element into its allocation gives the same bits in the input layer's weight
+    gradient (its operand is the caller's tensor; every sum it depends on runs in a fixed order)."""
+    print("[convae] gradient with an input aligned to one element", flush=True)
+    h = C.c_void_p()
+    check(lib().klrtm_convae_create(C.byref(h), 23))
+    n = lib().klrtm_convae_param_count()
+    x = np.random.default_rng(77).standard_normal(2 * 32768).astype(np.float32)
+    out = []
+    for shift in (0, 1, 3):
+        dx = DeviceArray.from_host(np.concatenate([np.zeros(shift, np.float32), x, np.zeros(4, np.float32)]))
+        g, loss = np.empty(n, np.float32), C.c_float()
+        check(lib().klrtm_convae_loss_grad(h.value, dx.ptr + 4 * shift, 2, g.ctypes.data, C.byref(loss)))
+        out.append(ref.split_params(g)[0][0])
+    lib().klrtm_convae_destroy(h.value)
+    assert all(np.array_equal(o.view(np.uint32), out[0].view(np.uint32)) for o in out)
