@@ -25,10 +25,11 @@
 // gathered from the input tensor per tap (im2col on the fly, zero outside the
 // grid), the B operand from weights pre-arranged in fragment order after every
 // update; the upsampling layers' and the output layer's forward have kernels of
-// their own (cae_up_kernel, cae_last_kernel).  Weight gradient: M = 32 output
-// channels, N = 32 (tap, input channel) pairs, K = positions, accumulated per
-// wave and added with FP32 atomics; the upsampling and the single-channel layers
-// again have their own (cae_wgrad_up_kernel, cae_wgrad_vec_kernel).
+// their own (cae_up_kernel, cae_last_kernel).  Weight gradient: M = 16 output
+// channels, N = 16 input channels (or taps), K = 32 positions, on
+// v_mfma_f32_16x16x32_bf16 from operands transposed into LDS as runs of 8
+// positions; partial sums of the workgroups are added in a fixed order
+// (cae_wgrad_up_kernel, cae_wgrad_vec_kernel, cae_wgrad_tile_kernel).
 // Training minimises the mean squared reconstruction error with Adam.
 #include "klrtm_internal.h"
 #include "convae.h"
@@ -462,9 +463,10 @@ __global__ void __launch_bounds__(512) cae_wgrad_up_kernel(const float *__restri
         o[(((ay * 4 + ax * 2 + az) * 8 + t) * COUT + c0 + q * 4 + r) * 32 + h * 16 + n] = acc[az][t][r];
 }
 
-// sum of nslot partial results of n values (n a multiple of 32) in a fixed order.  PITCH27: value i is
-// [i / 32][i % 32] of rows of 27 values in out.
-template<bool PITCH27>
+// sum of nslot partial results of n values (n a multiple of 32) in a fixed order.  R_PITCH27: value i is
+// [i / 32][i % 32] of rows of 27 values in out; R_TAPS: [tap][pair] of n / 27 pairs, out is [pair][tap].
+enum { R_PLAIN = 0, R_PITCH27 = 1, R_TAPS = 2 };
+template<int MODE>
 __global__ void __launch_bounds__(256) cae_wred_kernel(const float *__restrict__ part, int nslot, int n,
                                                        float *__restrict__ out) {
   __shared__ float s[256];
@@ -477,7 +479,8 @@ __global__ void __launch_bounds__(256) cae_wred_kernel(const float *__restrict__
   if(g) return;
 #pragma unroll
   for(int k = 1; k < 8; k++) v += s[k * 32 + l];
-  if(!PITCH27) out[i] = v;
+  if(MODE == R_PLAIN) out[i] = v;
+  else if(MODE == R_TAPS) out[i % (n / 27) * 27 + i / (n / 27)] = v;
   else if(l < 27) out[blockIdx.x * 27 + l] = v;
 }
 
@@ -502,7 +505,8 @@ __global__ void cae_wup_sum_kernel(const float *__restrict__ G, int cout, float 
 // D and S the 1-channel tensor on the 32^3 grid, at 2p + d (STRIDE 2) or p - d (STRIDE 1).  M = 16 channels, N = 27
 // taps in two halves, K = positions.  V is read once, straight into the operand; S lies in LDS three times, at the
 // three z offsets, as runs of 8 positions.  A workgroup walks slabs of 4 planes.  `part` as above: [slot][16][32].
-// 64 blocks, below 45 us each (gathered per tap and padded to 32 channels: 541 us and 1450 us).
+// 64 blocks: 8 us and 22 us, the latter for reading 134 MB of V (gathered per tap and padded to 32 channels: 541 us
+// and 1450 us).
 // (S may be the caller's tensor, aligned to its elements only: the hardware's wide loads accept that)
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 template<int LGP, int STRIDE>
@@ -552,8 +556,8 @@ __global__ void __launch_bounds__(256) cae_wgrad_vec_kernel(const float *__restr
     __syncthreads();
     const float *Vb = V + ((b << (3 * LGP)) + ((size_t)y0 << (2 * LGP))) * 16;
 #pragma unroll 4
-    for(int k = w; k < TY * D / RPK; k += 4) {
-      const int row = k * RPK + q / NCH, ch = q % NCH, ly = row >> LGP, x = row & (D - 1);
+    for(int k = 0; k < TY * D / RPK; k += 4) {
+      const int row = (k + w) * RPK + q / NCH, ch = q % NCH, ly = row >> LGP, x = row & (D - 1);
       const float *src = Vb + ((row << LGP) + ch * 8) * 16 + n;
       cae_bf16x8 a;
 #pragma unroll
@@ -575,52 +579,90 @@ __global__ void __launch_bounds__(256) cae_wgrad_vec_kernel(const float *__restr
     part[(size_t)blockIdx.x * 512 + i] = red[i] + red[512 + i] + red[1024 + i] + red[1536 + i];
 }
 
-// dW[co][ci][tap] += sum_{b, p} dZ[b][p][co] * X[b][q(p, tap)][ci] over a chunk of CAE_WG_CHUNK positions of
-// one block: M = output channels, N = 32 (tap, ci) pairs n = tap*CIN + ci, K = positions.  Long chunks keep
-// the atomic additions of the partial sums few (they all land on the layer's small dW).
-constexpr int CAE_WG_CHUNK = 4096;
-template<int CIN, int MODE>
-__global__ void __launch_bounds__(256) cae_wgrad_kernel(const float *__restrict__ X, const float *__restrict__ dZ,
-                                                        int cout, int lgo, int lgg, float *__restrict__ dW) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int Dout = 1 << lgo, Dg = 1 << lgg;
-  const long Pout = 1L << (3 * lgo), Pg = 1L << (3 * lgg);
-  const int n0 = (blockIdx.x * 4 + wv) * 32;
-  const long pc = (long)blockIdx.y * CAE_WG_CHUNK;
-  const long b = blockIdx.z;
-  if(n0 >= CIN * 27 || pc >= Pout) return;
-  const int half = lane >> 5, m = lane & 31;
-  const int n = n0 + (lane & 31), tap = n / CIN, ci = n - tap * CIN;
-  const int dy = tap / 9 - 1, dx = (tap / 3) % 3 - 1, dz = tap % 3 - 1;
-  const float *Xb = X + (size_t)b * Pg * CIN;
-  const float *Zb = dZ + (size_t)b * Pout * cout;
-  cae_f32x16 acc = {};
-  const long pend = pc + CAE_WG_CHUNK < Pout ? pc + CAE_WG_CHUNK : Pout;
-  for(long k0 = pc; k0 < pend; k0 += 16) {
-    cae_bf16x8 a, bb;
+// ---- weight gradients of the layers on the 8^3 grid ----------------------------------------------------
+//
+// dW[co][ci][tap] = sum_p dZ[p][co] X[STRIDE*p + d(tap)][ci] over the positions p of the 8^3 output grid.  As in
+// cae_wgrad_up_kernel both operands lie in LDS as runs of 8 z positions (here a whole row) of one channel, X three
+// times at the three z offsets.  A workgroup walks tiles of two planes; a wave owns 16 output channels, 16 input
+// channels and NT taps.  Columns past CIN and rows past COUT repeat the last channel and are not stored.
+// `part` is [slot][tap][co][ci].  64 blocks, one tile a workgroup: 12 us for 32 -> 32 and 10 us for 16 -> 32, bound by
+// the latency of one load, two barriers and the store of 108 KB of sums (32 taps and channels gathered per position from
+// L2 and added with atomics: 155 and 145 us).
+template<int CIN, int COUT, int STRIDE>
+__global__ void __launch_bounds__(512) cae_wgrad_tile_kernel(const float *__restrict__ X, const float *__restrict__ dZ,
+                                                             int ntask, float *__restrict__ part) {
+  constexpr int NI = (CIN + 15) / 16, NO = (COUT + 15) / 16, TG = 8 / (NI * NO), NT = (27 + TG - 1) / TG;
+  constexpr int DG = 8 * STRIDE, HX = STRIDE * 8 + 3 - STRIDE, HR = (STRIDE * 2 + 3 - STRIDE) * HX;
+  __shared__ __attribute__((aligned(16))) char xs[3 * HR * CIN * 16], zs[16 * COUT * 16];
+  const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, n = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), h = w % NI, c = w / NI % NO, g = w / (NI * NO);
+  int toff[NT];
 #pragma unroll
-    for(int t = 0; t < 8; t++) {
-      const long p = k0 + half * 8 + t;
-      float va = 0.f, vb = 0.f;
-      if(p < pend) {
-        if(m < cout) va = Zb[p * cout + m];
-        if(tap < 27) {
-          const int pz = (int)(p & (Dout - 1)), px = (int)((p >> lgo) & (Dout - 1)), py = (int)(p >> (2 * lgo));
-          const int qy = gather1(MODE, py, dy, Dout, Dg), qx = gather1(MODE, px, dx, Dout, Dg),
-                    qz = gather1(MODE, pz, dz, Dout, Dg);
-          if(qy >= 0 && qx >= 0 && qz >= 0) vb = Xb[(((((long)qy << lgg) + qx) << lgg) + qz) * CIN + ci];
-        }
+  for(int i = 0; i < NT; i++) {
+    const int tap = min(g * NT + i, 26), dy = tap / 9, dx = tap / 3 % 3, dz = tap % 3;
+    toff[i] = (dz * HR + dy * HX + dx) * CIN * 16;
+  }
+  const int ca = min(c * 16 + n, COUT - 1), cb = min(h * 16 + n, CIN - 1);
+  cae_f32x4 acc[NT] = {};
+  for(int task = blockIdx.x; task < ntask; task += gridDim.x) {
+    const size_t b = task >> 2;
+    const int y0 = (task & 3) * 2;
+    __syncthreads();  // the previous tile's products are done with the rows
+    for(int e = tid; e < HR * (CIN / 2); e += 512) {
+      const int cp = e % (CIN / 2), row = e / (CIN / 2), y = STRIDE * y0 + row / HX - 1, x = row % HX - 1;
+      const bool in = (unsigned)y < (unsigned)DG && (unsigned)x < (unsigned)DG;
+      const float *src = X + ((b * DG + (in ? y : 0)) * DG + (in ? x : 0)) * DG * CIN + cp * 2;
+      float2 v[DG];
+#pragma unroll
+      for(int k = 0; k < DG; k++) {
+        v[k] = *(const float2 *)(src + k * CIN);
+        if(!in) v[k] = float2{0.f, 0.f};
       }
-      a[t] = (__bf16)va, bb[t] = (__bf16)vb;
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bb, acc, 0, 0, 0);
-  }
-  if(tap >= 27) return;
 #pragma unroll
-  for(int r = 0; r < 16; r++) {
-    const int co = (r >> 2) * 8 + half * 4 + (r & 3);
-    if(co < cout) atomicAdd(&dW[((size_t)co * CIN + ci) * 27 + tap], acc[r]);
+      for(int o = 0; o < 3; o++) {
+        cae_bf16x8 s0, s1;
+#pragma unroll
+        for(int k = 0; k < 8; k++) {
+          const int z = STRIDE * k + o - 1;
+          const float2 f = z >= 0 && z < DG ? v[z < 0 ? 0 : z >= DG ? DG - 1 : z] : float2{0.f, 0.f};
+          s0[k] = (__bf16)f.x, s1[k] = (__bf16)f.y;
+        }
+        char *d = xs + ((o * HR + row) * CIN + cp * 2) * 16;
+        *(cae_bf16x8 *)d = s0, *(cae_bf16x8 *)(d + 16) = s1;
+      }
+    }
+    for(int e = tid; e < 16 * (COUT / 2); e += 512) {
+      const int cp = e % (COUT / 2), row = e / (COUT / 2);
+      const float *src = dZ + ((b * 64 + y0 * 8 + row) * 8) * COUT + cp * 2;
+      cae_bf16x8 s0, s1;
+#pragma unroll
+      for(int k = 0; k < 8; k++) {
+        const float2 f = *(const float2 *)(src + k * COUT);
+        s0[k] = (__bf16)f.x, s1[k] = (__bf16)f.y;
+      }
+      char *d = zs + (row * COUT + cp * 2) * 16;
+      *(cae_bf16x8 *)d = s0, *(cae_bf16x8 *)(d + 16) = s1;
+    }
+    __syncthreads();
+#pragma unroll
+    for(int ks = 0; ks < 4; ks++) {
+      const int row = ks * 4 + q, ly = row >> 3, lx = row & 7;
+      const cae_bf16x8 a = *(const cae_bf16x8 *)(zs + (row * COUT + ca) * 16);
+      const char *base = xs + ((STRIDE * ly * HX + STRIDE * lx) * CIN + cb) * 16;
+#pragma unroll
+      for(int i = 0; i < NT; i++)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, *(const cae_bf16x8 *)(base + toff[i]), acc[i], 0, 0, 0);
+    }
   }
+  float *o = part + (size_t)blockIdx.x * (27 * COUT * CIN);
+  const int ci = h * 16 + n;
+#pragma unroll
+  for(int i = 0; i < NT; i++)
+#pragma unroll
+    for(int r = 0; r < 4; r++) {
+      const int co = c * 16 + q * 4 + r;
+      if(g * NT + i < 27 && co < COUT && ci < CIN) o[((g * NT + i) * COUT + co) * CIN + ci] = acc[i][r];
+    }
 }
 
 // db[c] += sum over a chunk of positions of dZ[b][p][c]
@@ -1059,8 +1101,7 @@ static int layer_dgrad(const ConvAE &c, const CaeWork &w, int l, const float *dz
 
 // weight and bias gradients of layer l into d_grad (cleared before) from its input and its pre-activation gradient
 static int layer_wgrad(ConvAE &c, CaeWork &w, int l, const float *in, const float *dz, int nb) {
-  const int lgo = lg2(kDout[l]), lgg = lg2(kDin[l]);
-  const long P = 1L << (3 * lgo);
+  const long P = 1L << (3 * lg2(kDout[l]));
   float *dW = c.d_grad + c.w_off[l];
   const long n = (long)nb * P * kCout[l];
   hipLaunchKernelGGL(cae_bgrad_kernel, dim3((unsigned)((n + 8191) / 8192)), dim3(256), 0, stream(), dz, n, kCout[l],
@@ -1078,7 +1119,7 @@ static int layer_wgrad(ConvAE &c, CaeWork &w, int l, const float *in, const floa
       set_error("autoencoder layer %d has no weight-gradient kernel", l);
       return KLRTM_EINVAL;
     }
-    hipLaunchKernelGGL(cae_wred_kernel<false>, dim3((unsigned)(ng / 32)), dim3(256), 0, stream(), w.wpart, slots, ng, G);
+    hipLaunchKernelGGL(cae_wred_kernel<R_PLAIN>, dim3((unsigned)(ng / 32)), dim3(256), 0, stream(), w.wpart, slots, ng, G);
     hipLaunchKernelGGL(cae_wup_sum_kernel, dim3((unsigned)((kCout[l] * 32 * 27 + 255) / 256)), dim3(256), 0, stream(), G,
                        kCout[l], dW);
     return check_launch("cae_wgrad_up_kernel");
@@ -1090,22 +1131,23 @@ static int layer_wgrad(ConvAE &c, CaeWork &w, int l, const float *in, const floa
       hipLaunchKernelGGL((cae_wgrad_vec_kernel<4, 2>), dim3((unsigned)slots), dim3(256), 0, stream(), dz, in, ntask, w.wpart);
     else
       hipLaunchKernelGGL((cae_wgrad_vec_kernel<5, 1>), dim3((unsigned)slots), dim3(256), 0, stream(), in, dz, ntask, w.wpart);
-    hipLaunchKernelGGL(cae_wred_kernel<true>, dim3(16), dim3(256), 0, stream(), w.wpart, slots, 512, dW);
+    hipLaunchKernelGGL(cae_wred_kernel<R_PITCH27>, dim3(16), dim3(256), 0, stream(), w.wpart, slots, 512, dW);
     return check_launch("cae_wgrad_vec_kernel");
   }
-  const int ntile = (kCin[l] * 27 + 31) / 32;
-  const dim3 grid((unsigned)((ntile + 3) / 4), (unsigned)((P + CAE_WG_CHUNK - 1) / CAE_WG_CHUNK), (unsigned)nb);
-  const int mode = kKind[l] == K_DOWN ? G_DOWN : G_SAME;
-#define CAE_W(CI, M) \
-  hipLaunchKernelGGL((cae_wgrad_kernel<CI, M>), grid, dim3(256), 0, stream(), in, dz, kCout[l], lgo, lgg, dW)
-  switch(kCin[l] * 8 + mode) {
-  case 16 * 8 + G_DOWN: CAE_W(16, G_DOWN); break;
-  case 32 * 8 + G_SAME: CAE_W(32, G_SAME); break;
-  case 4 * 8 + G_SAME: CAE_W(4, G_SAME); break;
-  default: set_error("autoencoder layer %d has no weight-gradient kernel", l); return KLRTM_EINVAL;
+  const int nw = 27 * kCout[l] * kCin[l], ntask = nb * 4, slots = std::min(ntask, 256);
+#define CAE_W(CI, CO, S) \
+  hipLaunchKernelGGL((cae_wgrad_tile_kernel<CI, CO, S>), dim3((unsigned)slots), dim3(512), 0, stream(), in, dz, ntask, w.wpart)
+  if(kCin[l] == 16 && kCout[l] == 32 && kKind[l] == K_DOWN && kDout[l] == 8) CAE_W(16, 32, 2);
+  else if(kCin[l] == 32 && kCout[l] == 32 && kKind[l] == K_SAME && kDout[l] == 8) CAE_W(32, 32, 1);
+  else if(kCin[l] == 32 && kCout[l] == 4 && kKind[l] == K_SAME && kDout[l] == 8) CAE_W(32, 4, 1);
+  else if(kCin[l] == 4 && kCout[l] == 32 && kKind[l] == K_SAME && kDout[l] == 8) CAE_W(4, 32, 1);
+  else {
+    set_error("autoencoder layer %d has no weight-gradient kernel", l);
+    return KLRTM_EINVAL;
   }
 #undef CAE_W
-  return check_launch("cae_wgrad_kernel");
+  hipLaunchKernelGGL(cae_wred_kernel<R_TAPS>, dim3((unsigned)(nw / 32)), dim3(256), 0, stream(), w.wpart, slots, nw, dW);
+  return check_launch("cae_wgrad_tile_kernel");
 }
 
 // forward of layers [l0, l1) from in; pre-activations kept when training
