@@ -23,7 +23,7 @@ struct ConvAE {
   size_t wf_off[CAE_LAYERS] = {}, wb_off[CAE_LAYERS] = {};  // fragment offsets (16-byte units)
   float *d_param = nullptr, *d_grad = nullptr, *d_m = nullptr, *d_v = nullptr;  // FP32 master weights, Adam state
   void *d_wf = nullptr, *d_wb = nullptr;  // BF16 weight fragments: forward, data gradient
-  void *d_wu[CAE_LAYERS] = {};            // upsampling layers: phase fragments; last layer: tap fragment
+  void *d_wu[CAE_LAYERS] = {};            // tap fragments of the upsampling layers and of the last layer
   float *d_loss = nullptr;
   float h_loss[2] = {0.f, 0.f};
   int step = 0;

@@ -37,6 +37,7 @@
 #include <cmath>
 #include <cstring>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 namespace klrtm {
@@ -156,20 +157,20 @@ __global__ void __launch_bounds__(256) cae_conv_kernel(const float *__restrict__
 
 // ---- nearest x2 upsampling + 3x3x3 convolution, 32 -> COUT channels -----------------------------------
 //
-// A fine cell f = 2i + a (phase a in {0,1}^3) sees, along each axis, only the coarse cells i + t + a - 1, t in
-// {0,1}: the three taps of a phase fall on two coarse cells.  So a phase is a 2x2x2 convolution of the coarse grid
-// whose weights are sums of the layer's BF16-rounded weights.  A sum of up to eight is kept as two BF16 terms, its
-// rounding and the rest (2^-17 of it is lost; one rounded term moved a decoded volume by 0.8 %): 16 products a
-// phase instead of 27.
+// A fine cell f = 2i + a (phase a in {0,1}^3) sees, along each axis, the coarse cells i + t + a - 1 with t = 0 or 1:
+// tap d in {0, 1, 2} falls on t = (d > a).  Its 27 products are added in tap order, one v_mfma_f32_16x16x32_bf16 (a
+// tap's 32 channels) each: the same bits as two v_mfma_f32_32x32x16_bf16 a tap, the steps of the implicit GEMM.
+// (Sums of the weights that share a coarse cell would take 8 products instead of 27, but they do not fit BF16: one
+// rounded term moved a decoded volume by 0.8 %, two terms lose 2^-17 of each sum.)
 // One workgroup owns TY x TX x Dc coarse cells, staged with their halo as BF16 in LDS (pitch 80 bytes a cell: the
-// 16 cells of a fragment read fall on distinct banks).  A wave takes the two phases of one (ay, ax) at a time, for 16
-// output channels, keeps their 32 weight fragments in registers while it walks the tile's cells, and reads each
-// coarse cell's fragment once for both: 12 LDS reads for 32 matrix products v_mfma_f32_16x16x32_bf16.
+// 16 cells of a fragment read fall on distinct banks).  A wave keeps the 27 weight fragments of 16 output channels in
+// registers while it walks the tile's cells for one ay, one ax after the other, and forms both az at once: of a row
+// of taps it reads six coarse fragments and uses each for up to four of the 18 products.
+// 128 blocks: 178 us for layer 6 (46 us the matrix products, about 80 the vector instructions of 67 M exact GELUs,
+// 268 MB written) and 45 us for layer 5; gathering the taps per fine cell from L2, as the other layers do, the two
+// took 1364 us.
 // Operand layouts (lane l):
 //   A: A[l % 16][(l / 16)*8 + t]   B: B[(l / 16)*8 + t][l % 16]   C: register r holds C[(l / 16)*4 + r][l % 16]
-// 128 blocks: 161 us for layer 6 (about half of it the vector instructions of 67 M exact GELUs, 27 us the matrix
-// products, 268 MB written) and 42 us for layer 5; gathering 27 taps per fine cell from L2, as the other layers do,
-// the two took 1364 us.
 typedef float cae_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int CAE_UP_TY = 2, CAE_UP_TX = 8, CAE_UP_PITCH = 80;
 
@@ -185,53 +186,60 @@ __global__ void __launch_bounds__(256, 2) cae_up_kernel(const float *__restrict_
   static_assert(NYT * TY == Dc && NXT * TX == Dc, "whole tiles");
   const size_t b = blockIdx.y;
   const float *Xb = X + b * ((size_t)32 << (3 * LGD));
-  // stage the tile: four channels per thread and step
-  for(int e = threadIdx.x; e < CELLS * 8; e += 256) {
-    const int cell = e >> 3, c4 = (e & 7) * 4;
-    const int ly = cell / SX, r = cell - ly * SX, lx = r / SZ, lz = r - lx * SZ;
-    const int y = y0 + ly - 1, x = x0 + lx - 1, zz = lz - 1;
-    float4 v = {0.f, 0.f, 0.f, 0.f};
-    if((unsigned)y < (unsigned)Dc && (unsigned)x < (unsigned)Dc && (unsigned)zz < (unsigned)Dc)
-      v = *(const float4 *)(Xb + (size_t)(((y << LGD) + x) << LGD) * 32 + zz * 32 + c4);
-    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-    bf4 h;
-    h[0] = (__bf16)v.x, h[1] = (__bf16)v.y, h[2] = (__bf16)v.z, h[3] = (__bf16)v.w;
-    *(bf4 *)(lds + cell * CAE_UP_PITCH + c4 * 2) = h;
+  // stage the tile: four channels per thread and step, eight steps' loads in flight
+  typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+  constexpr int U = 8;
+  for(int e0 = threadIdx.x; e0 < CELLS * 8; e0 += 256 * U) {
+    float4 v[U];
+#pragma unroll
+    for(int u = 0; u < U; u++) {
+      const int e = e0 + 256 * u, cell = e >> 3, c4 = (e & 7) * 4;
+      const int ly = cell / SX, r = cell - ly * SX, lx = r / SZ, lz = r - lx * SZ;
+      const int y = y0 + ly - 1, x = x0 + lx - 1, zz = lz - 1;
+      v[u] = float4{0.f, 0.f, 0.f, 0.f};
+      if(e < CELLS * 8 && (unsigned)y < (unsigned)Dc && (unsigned)x < (unsigned)Dc && (unsigned)zz < (unsigned)Dc)
+        v[u] = *(const float4 *)(Xb + (size_t)(((y << LGD) + x) << LGD) * 32 + zz * 32 + c4);
+    }
+#pragma unroll
+    for(int u = 0; u < U; u++) {
+      const int e = e0 + 256 * u;
+      bf4 h;
+      h[0] = (__bf16)v[u].x, h[1] = (__bf16)v[u].y, h[2] = (__bf16)v[u].z, h[3] = (__bf16)v[u].w;
+      if(e < CELLS * 8) *(bf4 *)(lds + (e >> 3) * CAE_UP_PITCH + (e & 7) * 8) = h;
+    }
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, n = lane & 15;
-  // two passes: COUT 32: wave = (ay, ax), pass = half of the channels; COUT 16: wave = (ay, every second row of
-  // cells), pass = ax
+  // wave = (ay, half of the channels) of 32 channels, (ay, every second row of cells) of 16
   constexpr int NT = COUT / 16, RPM = Dc == 8 ? 2 : 1, MT = TY * TX / RPM;  // 16 cells: one row of 16 or two of 8
+  const int ay = w & 1, h = NT == 2 ? w >> 1 : 0;
+  cae_bf16x8 B[27];
+#pragma unroll
+  for(int t = 0; t < 27; t++) B[t] = wu[(t * NT + h) * 64 + lane];
+  const float bn = bias[h * 16 + n];
   __syncthreads();
-  for(int pass = 0; pass < 2; pass++) {
-    const int ay = COUT == 32 ? w >> 1 : w & 1, ax = COUT == 32 ? w & 1 : pass, h = COUT == 32 ? pass : 0;
-    cae_bf16x8 B[2][8][2];  // [az][t][rounded, rest]
-#pragma unroll
-    for(int az = 0; az < 2; az++)
-#pragma unroll
-      for(int t = 0; t < 8; t++)
-#pragma unroll
-        for(int k = 0; k < 2; k++) B[az][t][k] = wu[(((((ay * 2 + ax) * 2 + az) * 8 + t) * NT + h) * 2 + k) * 64 + lane];
-    const float bn = bias[h * 16 + n];
-    for(int m = COUT == 32 ? 0 : w >> 1; m < MT; m += COUT == 32 ? 1 : 2) {
+  auto phases = [&](auto ax_tag) __attribute__((always_inline)) {
+    constexpr int ax = decltype(ax_tag)::value;
+    for(int m = NT == 2 ? 0 : w >> 1; m < MT; m += 3 - NT) {
       const int row = m * RPM + (Dc == 8 ? n >> 3 : 0), ly = row / TX, lx = row % TX, lz = n & (Dc - 1);
       const char *base = lds + ((ly + ay) * SX + (lx + ax) * SZ + lz) * CAE_UP_PITCH + q * 16;
       cae_f32x4 acc[2] = {};
 #pragma unroll
-      for(int ty = 0; ty < 2; ty++)
+      for(int dy = 0; dy < 3; dy++) {
+        const char *by = base + (dy == 0 || (dy == 1 && ay) ? 0 : SX * CAE_UP_PITCH);
+        cae_bf16x8 A[2][3];  // coarse x offset t, z offset - 1
 #pragma unroll
-        for(int tx = 0; tx < 2; tx++)
+        for(int t = 0; t < 2; t++)
 #pragma unroll
-          for(int oz = 0; oz < 3; oz++) {  // coarse z offset oz - 1: tap oz - az of phase az
-            const cae_bf16x8 a = *(const cae_bf16x8 *)(base + (ty * SX + tx * SZ + oz) * CAE_UP_PITCH);
+          for(int o = 0; o < 3; o++) A[t][o] = *(const cae_bf16x8 *)(by + (t * SZ + o) * CAE_UP_PITCH);
 #pragma unroll
-            for(int az = 0; az < 2; az++) {
-              if(oz - az < 0 || oz - az > 1) continue;
+        for(int dx = 0; dx < 3; dx++)
 #pragma unroll
-              for(int k = 0; k < 2; k++)
-                acc[az] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, B[az][(ty * 2 + tx) * 2 + oz - az][k], acc[az], 0, 0, 0);
-            }
-          }
+          for(int dz = 0; dz < 3; dz++)
+#pragma unroll
+            for(int az = 0; az < 2; az++)
+              acc[az] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[dx > ax][(dz > az) + az], B[(dy * 3 + dx) * 3 + dz],
+                                                                acc[az], 0, 0, 0);
+      }
 #pragma unroll
       for(int r = 0; r < 4; r++) {
         const int mr = q * 4 + r, rr = m * RPM + (Dc == 8 ? mr >> 3 : 0);
@@ -246,113 +254,113 @@ __global__ void __launch_bounds__(256, 2) cae_up_kernel(const float *__restrict_
         }
       }
     }
-  }
+  };
+  phases(std::integral_constant<int, 0>());
+  phases(std::integral_constant<int, 1>());
 }
 
-// phase fragments of an upsampling layer: wu[((ay, ax, az), (ty, tx, tz), half, rounded / rest)][lane], k = input
-// channel
+// weight fragments of an upsampling layer: wu[tap][half of the channels][lane], k = input channel
 __global__ void cae_wup_kernel(const float *__restrict__ W, int cout, cae_bf16x8 *__restrict__ wu) {
   const int nt = cout / 16, i = blockIdx.x * blockDim.x + threadIdx.x;
-  if(i >= 64 * nt * 64) return;
-  const int l = i & 63, h = (i >> 6) % nt, t = (i >> 6) / nt % 8, a = (i >> 6) / nt / 8;
-  const int co = h * 16 + (l & 15);
-  // taps d (0..2 for -1..1) of phase bit p that fall on coarse offset t + p - 1: p = 0: {0}, {1, 2}; p = 1: {0, 1}, {2}
-  auto lo = [](int p, int tt) { return tt == 0 ? 0 : p == 0 ? 1 : 2; };
-  auto hi = [](int p, int tt) { return tt == 1 ? 2 : p == 0 ? 0 : 1; };
-  const int ay = a >> 2, ax = (a >> 1) & 1, az = a & 1, ty = t >> 2, tx = (t >> 1) & 1, tz = t & 1;
-  cae_bf16x8 v, r;
+  if(i >= 27 * nt * 64) return;
+  const int l = i & 63, co = (i >> 6) % nt * 16 + (l & 15), tap = (i >> 6) / nt;
+  cae_bf16x8 v;
 #pragma unroll
-  for(int j = 0; j < 8; j++) {
-    const int ci = (l >> 4) * 8 + j;
-    float s = 0.f;
-    for(int dy = lo(ay, ty); dy <= hi(ay, ty); dy++)
-      for(int dx = lo(ax, tx); dx <= hi(ax, tx); dx++)
-        for(int dz = lo(az, tz); dz <= hi(az, tz); dz++) s += (float)(__bf16)W[((size_t)co * 32 + ci) * 27 + (dy * 3 + dx) * 3 + dz];
-    v[j] = (__bf16)s;
-    r[j] = (__bf16)(s - (float)v[j]);
-  }
-  const size_t o = ((size_t)(i >> 6) * 2) * 64 + l;
-  wu[o] = v, wu[o + 64] = r;
+  for(int j = 0; j < 8; j++) v[j] = (__bf16)W[((size_t)co * 32 + (l >> 4) * 8 + j) * 27 + tap];
+  wu[i] = v;
 }
 
 // ---- the output layer: 3x3x3 convolution of 16 channels to one on the 32^3 grid ------------------------
 //
-// First the products of every cell with all 27 taps, T[cell][tap] = sum_c x[cell][c] W[tap][c] (one
-// v_mfma_f32_32x32x16_bf16 per row of 32 cells: taps are the columns), then y[p] = sum_tap T[p + d(tap)][tap] from LDS.
-// As an ordinary implicit GEMM one of 32 columns did useful work and every cell's channels were gathered 27 times
-// (513 us for 128 blocks, now 58 us).  A workgroup owns 8 rows (and one more on each side) and walks along y; each thread keeps
-// the three output planes its cell contributes to.
+// The cells are the columns, 16 along z, and the weights row 0 of the other operand: a v_mfma_f32_16x16x32_bf16 adds
+// two taps' channels, in tap order and with the bits of the implicit GEMM's one tap a step (a 28th tap is zero on
+// both sides).  15 of 16 rows are padding; sums over each cell's products with all taps, which need none, round
+// every tap's product sum to FP32 before it is added.
+// 128 blocks: 71 us, bound by the LDS reads (48 us) and the 268 MB read (55 us at the copy rate); as an ordinary
+// implicit GEMM, which gathers every cell's channels 27 times from L2, 513 us.
+// A workgroup owns 8 rows (and one more on each side) and walks along y with three planes and the next one as BF16
+// in LDS, channel halves apart: [half][row][z], 16 bytes each, so a fragment read is contiguous.
+constexpr int CAE_LT = 14;  // steps of two taps
 __global__ void cae_wtap_kernel(const float *__restrict__ W, cae_bf16x8 *__restrict__ wt) {
-  const int l = threadIdx.x, tap = l & 31;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if(i >= CAE_LT * 64) return;
+  const int l = i & 63, q = l >> 4, tap = (i >> 6) * 2 + (q >> 1);
   cae_bf16x8 v;
 #pragma unroll
-  for(int j = 0; j < 8; j++) v[j] = (__bf16)(tap < 27 ? W[((l >> 5) * 8 + j) * 27 + tap] : 0.f);
-  wt[l] = v;
+  for(int j = 0; j < 8; j++) v[j] = (__bf16)((l & 15) == 0 && tap < 27 ? W[((q & 1) * 8 + j) * 27 + tap] : 0.f);
+  wt[i] = v;
 }
 __global__ void __launch_bounds__(256) cae_last_kernel(const float *__restrict__ X, const cae_bf16x8 *__restrict__ wt,
                                                        const float *__restrict__ bias, float *__restrict__ out) {
-  constexpr int ROWS = 10;
-  __shared__ float T[ROWS * 32 * 27];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  constexpr int ROWS = 10, SX = 34, HALF = ROWS * SX, PLANE = 2 * HALF;  // in 16-byte units
+  __shared__ cae_bf16x8 T[4 * PLANE];                                    // plane y in slot y & 3
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, n = lane & 15;
   const int x0 = blockIdx.x * 8;
   const size_t b = blockIdx.y;
   const float *Xb = X + b * (32768 * 16);
-  const cae_bf16x8 B = wt[lane];
-  const int lx = threadIdx.x >> 5, lz = threadIdx.x & 31;  // this thread's output column
-  float o0 = bias[0], o1 = o0, o2;  // outputs of planes y-1, y, y+1
-  // rows w, w + 4, w + 8 of plane y
-  auto load = [&](int y, float4(&v)[3][2]) __attribute__((always_inline)) {
+  cae_bf16x8 W[CAE_LT];
 #pragma unroll
-    for(int k = 0; k < 3; k++) {
-      const int r = w + 4 * k, x = x0 + r - 1;
+  for(int s = 0; s < CAE_LT; s++) W[s] = wt[s * 64 + lane];
+  const float b0 = bias[0];
+  const cae_bf16x8 zero = {};
+  // 640 items a plane: 8 channels of one cell
+  constexpr int NI = 3;
+  float4 v[NI][2];
+  auto load = [&](int y) __attribute__((always_inline)) {
+#pragma unroll
+    for(int k = 0; k < NI; k++) {
+      const int e = tid + k * 256, hf = e & 1, z = (e >> 1) & 31, x = x0 + (e >> 6) - 1;
       v[k][0] = v[k][1] = float4{0.f, 0.f, 0.f, 0.f};
-      if(r < ROWS && (unsigned)x < 32u && y < 32) {
-        const float4 *src = (const float4 *)(Xb + (((size_t)y * 32 + x) * 32 + (lane & 31)) * 16 + (lane >> 5) * 8);
+      if(e < ROWS * 64 && (unsigned)x < 32u && (unsigned)y < 32u) {
+        const float4 *src = (const float4 *)(Xb + (((size_t)y * 32 + x) * 32 + z) * 16 + hf * 8);
         v[k][0] = src[0], v[k][1] = src[1];
       }
     }
   };
-  float4 v[3][2];
-  load(0, v);
-  for(int y = 0; y < 32; y++) {
-    cae_f32x16 acc[3];
+  auto put = [&](int y) __attribute__((always_inline)) {
 #pragma unroll
-    for(int k = 0; k < 3; k++) {
+    for(int k = 0; k < NI; k++) {
+      const int e = tid + k * 256, hf = e & 1, z = (e >> 1) & 31, r = e >> 6;
+      if(e >= ROWS * 64) continue;
       cae_bf16x8 a;
       a[0] = (__bf16)v[k][0].x, a[1] = (__bf16)v[k][0].y, a[2] = (__bf16)v[k][0].z, a[3] = (__bf16)v[k][0].w;
       a[4] = (__bf16)v[k][1].x, a[5] = (__bf16)v[k][1].y, a[6] = (__bf16)v[k][1].z, a[7] = (__bf16)v[k][1].w;
-      acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B, cae_f32x16{}, 0, 0, 0);
+      T[(y & 3) * PLANE + hf * HALF + r * SX + z + 1] = a;
     }
-    load(y + 1, v);
-    __syncthreads();  // the sums of plane y-1 are done with T
-    const int tap = lane & 31;
-    if(tap < 27) {
-#pragma unroll
-      for(int k = 0; k < 3; k++)
-        if(w + 4 * k < ROWS) {
-#pragma unroll
-          for(int r = 0; r < 16; r++)
-            T[((w + 4 * k) * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * 27 + tap] = acc[k][r];
-        }
-    }
+  };
+  // the cells beside z = 0 and 31 stay zero
+  for(int e = tid; e < 4 * 2 * ROWS * 2; e += 256) T[(e >> 1) * SX + (e & 1) * (SX - 1)] = zero;
+  load(-1), put(-1);
+  load(0), put(0);
+  load(1);
+  for(int y = 0; y < 32; y++) {
+    put(y + 1);  // into the slot of plane y - 3, which every wave left before the barrier of y - 1
+    load(y + 2);
     __syncthreads();
-    // y[p] += T[p + d][tap(d)]: plane y is d_y = +1 of output y-1, 0 of y, -1 of y+1
-    float s[3] = {0.f, 0.f, 0.f};
+    // four runs of 16 cells a wave, rows lx, lx + 2, ..: this lane's channel half of cell z0 + n, tap offset (-1, -1, -1)
+    const int lx = w >> 1, z0 = (w & 1) * 16;
+    const cae_bf16x8 *base = T + (q & 1) * HALF + lx * SX + z0 + n;
+    cae_f32x4 acc[4] = {};
+    cae_bf16x8 keep[4];  // a pair two rows on is the next run's pair three steps before
 #pragma unroll
-    for(int dx = 0; dx < 3; dx++)
+    for(int s = 0; s < CAE_LT; s++) {
+      const bool first = s == 0 || s == 5 || s == 9, again = s == 3 || s == 8 || s == 12;
+      const int t0 = 2 * s, t1 = 2 * s + 1;
+      auto off = [&](int t) { return ((y + t / 9 - 1) & 3) * PLANE + t / 3 % 3 * SX + t % 3; };
+      const cae_bf16x8 *p = base + (q >> 1 && t1 < 27 ? off(t1) : off(t0));
 #pragma unroll
-      for(int dz = 0; dz < 3; dz++) {
-        const int zz = lz + dz - 1;
-        const float *t = T + ((lx + dx) * 32 + min(max(zz, 0), 31)) * 27 + dx * 3 + dz;
-        const bool ok = (unsigned)zz < 32u;
-#pragma unroll
-        for(int dy = 0; dy < 3; dy++) s[dy] += ok ? t[dy * 9] : 0.f;
+      for(int u = 0; u < 4; u++) {
+        cae_bf16x8 a = again && u < 3 ? keep[u + 1] : p[2 * u * SX];
+        if(first) keep[u] = a;
+        if(t1 == 27) a = q >> 1 ? zero : a;
+        acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[s], a, acc[u], 0, 0, 0);
       }
-    o0 += s[2], o1 += s[1], o2 = bias[0] + s[0];
-    if(y > 0) out[b * 32768 + ((size_t)(y - 1) * 32 + x0 + lx) * 32 + lz] = o0;
-    o0 = o1, o1 = o2;
+    }
+    if(lane < 16) {
+#pragma unroll
+      for(int u = 0; u < 4; u++) out[b * 32768 + ((size_t)y * 32 + x0 + lx + 2 * u) * 32 + z0 + lane] = acc[u][0] + b0;
+    }
   }
-  out[b * 32768 + ((size_t)31 * 32 + x0 + lx) * 32 + lz] = o0;
 }
 
 // ---- weight gradients of the upsampling layers ---------------------------------------------------------
@@ -944,8 +952,8 @@ int cae_create(ConvAE **out, unsigned seed) {
   if(e == hipSuccess) e = hipMalloc(&c->d_wf, foff * sizeof(cae_bf16x8));
   if(e == hipSuccess) e = hipMalloc(&c->d_wb, boff * sizeof(cae_bf16x8));
   for(int l = 0; l < CAE_LAYERS && e == hipSuccess; l++)
-    if(kKind[l] == K_UP) e = hipMalloc(&c->d_wu[l], (size_t)64 * (kCout[l] / 16) * 2 * 64 * sizeof(cae_bf16x8));
-    else if(l == CAE_LAYERS - 1) e = hipMalloc(&c->d_wu[l], 64 * sizeof(cae_bf16x8));
+    if(kKind[l] == K_UP) e = hipMalloc(&c->d_wu[l], (size_t)27 * (kCout[l] / 16) * 64 * sizeof(cae_bf16x8));
+    else if(l == CAE_LAYERS - 1) e = hipMalloc(&c->d_wu[l], (size_t)CAE_LT * 64 * sizeof(cae_bf16x8));
   if(e == hipSuccess) e = hipMalloc(&c->d_loss, sizeof(float) * 2);
   if(e == hipSuccess) e = hipMemcpy(c->d_param, h.data(), off * 4, hipMemcpyHostToDevice);
   if(e == hipSuccess) e = hipMemset(c->d_m, 0, off * 4);
@@ -971,10 +979,10 @@ int cae_refresh(ConvAE &c) {
     hipLaunchKernelGGL(cae_wfrag_kernel, dim3((n + 255) / 256), dim3(256), 0, stream(), c.d_param + c.w_off[l], kCin[l],
                        kCout[l], ksf, ksb, (cae_bf16x8 *)c.d_wf + c.wf_off[l], (cae_bf16x8 *)c.d_wb + c.wb_off[l]);
     if(kKind[l] == K_UP)
-      hipLaunchKernelGGL(cae_wup_kernel, dim3(kCout[l] / 16 * 16), dim3(256), 0, stream(), c.d_param + c.w_off[l], kCout[l],
+      hipLaunchKernelGGL(cae_wup_kernel, dim3((27 * 64 * (kCout[l] / 16) + 255) / 256), dim3(256), 0, stream(), c.d_param + c.w_off[l], kCout[l],
                          (cae_bf16x8 *)c.d_wu[l]);
     else if(l == CAE_LAYERS - 1)
-      hipLaunchKernelGGL(cae_wtap_kernel, dim3(1), dim3(64), 0, stream(), c.d_param + c.w_off[l], (cae_bf16x8 *)c.d_wu[l]);
+      hipLaunchKernelGGL(cae_wtap_kernel, dim3((CAE_LT * 64 + 255) / 256), dim3(256), 0, stream(), c.d_param + c.w_off[l], (cae_bf16x8 *)c.d_wu[l]);
   }
   return check_launch("cae_wfrag_kernel");
 }
