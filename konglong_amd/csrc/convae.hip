@@ -216,10 +216,13 @@ __global__ void __launch_bounds__(256, 2) cae_up_kernel(const float *__restrict_
 #pragma unroll
   for(int t = 0; t < 27; t++) B[t] = wu[(t * NT + h) * 64 + lane];
   const float bn = bias[h * 16 + n];
+  // a workgroup of several for a tile takes one ax and every (parts / 2)-th of the wave's rows
+  const int parts = gridDim.z, part = blockIdx.z, rs = parts > 2 ? parts >> 1 : 1;
+  const int m0 = (NT == 2 ? 0 : w >> 1) + (3 - NT) * (part >> 1), dm = (3 - NT) * rs;
   __syncthreads();
   auto phases = [&](auto ax_tag) __attribute__((always_inline)) {
     constexpr int ax = decltype(ax_tag)::value;
-    for(int m = NT == 2 ? 0 : w >> 1; m < MT; m += 3 - NT) {
+    for(int m = m0; m < MT; m += dm) {
       const int row = m * RPM + (Dc == 8 ? n >> 3 : 0), ly = row / TX, lx = row % TX, lz = n & (Dc - 1);
       const char *base = lds + ((ly + ay) * SX + (lx + ax) * SZ + lz) * CAE_UP_PITCH + q * 16;
       cae_f32x4 acc[2] = {};
@@ -255,8 +258,8 @@ __global__ void __launch_bounds__(256, 2) cae_up_kernel(const float *__restrict_
       }
     }
   };
-  phases(std::integral_constant<int, 0>());
-  phases(std::integral_constant<int, 1>());
+  if(parts == 1 || !(part & 1)) phases(std::integral_constant<int, 0>());
+  if(parts == 1 || part & 1) phases(std::integral_constant<int, 1>());
 }
 
 // weight fragments of an upsampling layer: wu[tap][half of the channels][lane], k = input channel
@@ -295,7 +298,7 @@ __global__ void __launch_bounds__(256) cae_last_kernel(const float *__restrict__
   constexpr int ROWS = 10, SX = 34, HALF = ROWS * SX, PLANE = 2 * HALF;  // in 16-byte units
   __shared__ cae_bf16x8 T[4 * PLANE];                                    // plane y in slot y & 3
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, n = lane & 15;
-  const int x0 = blockIdx.x * 8;
+  const int x0 = (blockIdx.x & 3) * 8, planes = 128 / gridDim.x, y0 = (blockIdx.x >> 2) * planes;
   const size_t b = blockIdx.y;
   const float *Xb = X + b * (32768 * 16);
   cae_bf16x8 W[CAE_LT];
@@ -330,12 +333,12 @@ __global__ void __launch_bounds__(256) cae_last_kernel(const float *__restrict__
   };
   // the cells beside z = 0 and 31 stay zero
   for(int e = tid; e < 4 * 2 * ROWS * 2; e += 256) T[(e >> 1) * SX + (e & 1) * (SX - 1)] = zero;
-  load(-1), put(-1);
-  load(0), put(0);
-  load(1);
-  for(int y = 0; y < 32; y++) {
+  load(y0 - 1), put(y0 - 1);
+  load(y0), put(y0);
+  load(y0 + 1);
+  for(int y = y0; y < y0 + planes; y++) {
     put(y + 1);  // into the slot of plane y - 3, which every wave left before the barrier of y - 1
-    load(y + 2);
+    if(y + 1 < y0 + planes) load(y + 2);
     __syncthreads();
     // four runs of 16 cells a wave, rows lx, lx + 2, ..: this lane's channel half of cell z0 + n, tap offset (-1, -1, -1)
     const int lx = w >> 1, z0 = (w & 1) * 16;
@@ -1036,6 +1039,16 @@ static void conv_launch(const float *G, const void *wf, int ks, int nout, int lg
                      lgo, lgg, bias, act, z, out, zg);
 }
 
+// Workgroups that share a tile of the upsampling layers, and slabs along y of the output layer's columns, for a launch
+// of wg tiles: up to two workgroups a CU, past which the repeated staging costs more than it hides.  1, 8, 27 and 64
+// blocks, us with 1 / 2 / 4 / 8 parts: layer 6 34 22 16 14, 39 28 24 30, 47 56 70 96, 91 109 148 226; layer 5 29 19 13 10,
+// 30 19 14 11, 32 21 17 22, 36 28 31 35; output layer 50 27 15 9, 50 27 16 11, 51 29 23 27, 54 41 48 48.
+static int cae_parts(long wg) {
+  int parts = 1;
+  while(parts < 8 && 2 * wg * parts <= 512) parts *= 2;
+  return parts;
+}
+
 // forward of layer l over nb blocks: out = act(conv(in) + b), pre-activation kept in z when set
 static int layer_fwd(const ConvAE &c, int l, const float *in, float *z, float *out, int nb) {
   const int lgo = lg2(kDout[l]), lgg = lg2(kDin[l]), ks = ksteps(kCin[l]);
@@ -1044,7 +1057,7 @@ static int layer_fwd(const ConvAE &c, int l, const float *in, float *z, float *o
   const cae_bf16x8 *wu = (const cae_bf16x8 *)c.d_wu[l];
   if(kKind[l] == K_UP) {
     const int tiles = (kDin[l] / CAE_UP_TY) * (kDin[l] / CAE_UP_TX);
-    const dim3 grid((unsigned)tiles, (unsigned)nb);
+    const dim3 grid((unsigned)tiles, (unsigned)nb, (unsigned)cae_parts((long)tiles * nb));
     if(kCout[l] == 32 && kDin[l] == 8)
       hipLaunchKernelGGL((cae_up_kernel<32, 3>), grid, dim3(256), 0, stream(), in, wu, bias, z, out);
     else if(kCout[l] == 16 && kDin[l] == 16)
@@ -1056,7 +1069,8 @@ static int layer_fwd(const ConvAE &c, int l, const float *in, float *z, float *o
     return check_launch("cae_up_kernel");
   }
   if(l == CAE_LAYERS - 1) {  // (no activation: nothing reads its pre-activation)
-    hipLaunchKernelGGL(cae_last_kernel, dim3(4, (unsigned)nb), dim3(256), 0, stream(), in, wu, bias, out);
+    hipLaunchKernelGGL(cae_last_kernel, dim3(4 * (unsigned)cae_parts(4L * nb), (unsigned)nb), dim3(256), 0, stream(), in, wu,
+                       bias, out);
     return check_launch("cae_last_kernel");
   }
   const int mode = kKind[l] == K_DOWN ? G_DOWN : G_SAME;

@@ -38,3 +38,19 @@ def test_no_bit_of_a_weight_sum_is_lost(klrtm, layer, taps):
     got = rec.download()[:, 2:-2, 2:-2, 2:-2]  # cells whose taps all lie inside the layer's output grid
     want = 2.0 ** (-17 if layer == 6 else -18)
     assert np.all(np.abs(got - want) < 1e-3 * want), (float(got.min()) / want, float(got.max()) / want)
+
+
+@pytest.mark.parametrize("nb", [5, 9, 17, 33, 65])
+def test_a_block_does_not_depend_on_the_batch(klrtm, nb):
+    """How many workgroups share a tile follows from the number of blocks (8 for one block; with these numbers every
+    other choice of the three layers); each output's products are added in the same order all the same."""
+    print(f"[convae] {nb} blocks at once and one by one", flush=True)
+    h = C.c_void_p()
+    check(lib().klrtm_convae_create(C.byref(h), 31))
+    x = np.random.default_rng(nb).standard_normal((nb, 32, 32, 32)).astype(np.float32)
+    dx, rec, one = DeviceArray.from_host(x), DeviceArray(x.shape), DeviceArray(x.shape)
+    check(lib().klrtm_convae_forward(h.value, dx.ptr, nb, None, rec.ptr))
+    for b in range(nb):
+        check(lib().klrtm_convae_forward(h.value, dx.ptr + b * 131072, 1, None, one.ptr + b * 131072))
+    lib().klrtm_convae_destroy(h.value)
+    assert np.array_equal(rec.download().view(np.uint32), one.download().view(np.uint32))
