@@ -256,34 +256,42 @@ int Engine::set_boundary(const int *nbnd, float dt_, float vmax_) {
 }
 
 // Effective tile: the values set through klrtm_kernel_set_tile, the defaults for the rest: 64 z lanes (one
-// wave per x row) by 8 x rows, and the y chunk whose blocks load the 256 CUs most evenly.  A launch takes about
-// (blocks on the fullest CU + 1) * (planes of a block + 3R): a block's start costs R halo planes on each side and
-// the latency of its first loads, and the last block of a CU runs alone.  At least two blocks a CU where the
-// grid has them.  Sweeps of the chunk (MI355X): TTI FD16 300^3 75 planes (0.79 ms a step; 150 planes 0.93, 32
-// planes 0.91), TTI FD16 600x600x400 150 (3.67; 300: 3.91, 60: 3.93), ISO FD8 400^3 67-100 (0.383; 200: 0.441),
-// ISO FD8 128^3 8 (19.6 us; 16: 22.1, 22: 27), VTI FD8 50x55x60 1-2 (20 us; 32 planes 88 us).
-void Engine::default_tile(int R, int &etz, int &etx, int &eyc) const {
+// wave per x row) by 8 x rows, and the y chunk whose blocks load the 256 CUs most evenly.
+// A launch takes about (k + w * rounds) * (chunk + h), k the blocks on the fullest CU, h the planes' time that a
+// block's halo planes and first loads cost, and w the planes' time of waiting per plane of a round of resident
+// blocks, which only a second resident block fills.  Where a CU holds two workgroups of 8 waves (kernels of <= 128
+// VGPRs: the Laplacian up to FD12, both first-derivative passes up to FD10; one of the two up to FD12, and up to FD16
+// in VTI) h is R / 2 and w 1.5 (one pass of two: 0.5), and past two blocks a CU the blocks partly even out by
+// themselves (x, the mean, has its share beside k); where it holds one, h is 10 and w 0.1.
+// Sweeps of every chunk over ISO FD8, 10, 12, 16 and VTI and TTI FD8, 12, 16 on 18 grids from 40x44x48 to
+// 600x600x400 (MI355X) gave the constants: the rule's chunk takes 1.005 times the best one's time in the mean and
+// 1.08 times at worst (TTI FD8 350x310x370: 0.90 ms, with 11 planes 0.84; ISO at most 1.03).  Asking for 512 blocks
+// whatever the chunk took up to 1.68 times (ISO FD16 80^3, 3 planes: 27.7 us, 7 planes 16.9; 96^3 29.1 and 20.6;
+// 128^3 32.7 and 27.5), chunks of at least 2R planes up to 2.8 times (ISO FD16 48^3 25.6 and 9.6 us).
+void Engine::default_tile(int R, bool first_deriv, bool tti, int &etz, int &etx, int &eyc) const {
   etz = tz > 0 ? tz : std::max(R, std::min(64, nz));
   etx = tx > 0 ? tx : std::max(R, 8);
   while(etz * etx > 512) etx = std::max(R, etx / 2);  // the stencil kernels are built for <= 512 threads
   eyc = ychunk;
   if(eyc > 0) return;
-  const long tiles = (long)div_up(nz, etz) * div_up(nx, etx);
-  const bool two = tiles * ny >= 512;
-  long best = 0;
-  for(int n = 1; n <= ny; n++) {
-    const int chunk = div_up(ny, n);
-    const long blocks = tiles * div_up(ny, chunk);
-    if(two && blocks < 512) continue;
-    const long cost = (div_up(blocks, 256) + 1L) * (chunk + 3 * R);
+  const bool one = R >= 7 && (!first_deriv || tti);
+  const double w = one ? 0.1 : !first_deriv || R <= 5 ? 1.5 : 0.5, h = one ? 10. : 0.5 * R;
+  const double tiles = (double)div_up(nz, etz) * div_up(nx, etx) / (256 * std::max(1, 512 / (etz * etx)));
+  double best = 0.;
+  for(int chunk = ny;;) {  // the chunks that cut ny into 1, 2, .. parts, each once
+    const double x = tiles * div_up(ny, chunk), k = std::ceil(x);
+    const double rounds = std::ceil(0.5 * k);
+    const double cost = (one || k <= 2. ? k + w * rounds : 0.4 * k + 0.6 * x + w * (0.25 * rounds + 0.375 * x)) * (chunk + h);
     if(eyc <= 0 || cost < best) best = cost, eyc = chunk;
+    if(chunk == 1) break;
+    chunk = div_up(ny, div_up(ny, chunk - 1));
   }
 }
 
-void Engine::fill_args(IsoArgs &a, int deriv_order) {
+void Engine::fill_args(IsoArgs &a, int deriv_order, int model) {
   memset(&a, 0, sizeof(a));
   a.nx = nx, a.ny = ny, a.nz = nz;
-  default_tile(ne, a.tz, a.tx, a.ychunk);
+  default_tile(ne, deriv_order == 1, model == KLRTM_TTI, a.tz, a.tx, a.ychunk);
   a.do_y = ny > 2;
   a.has_pml = has_pml;
   a.pml = desc;
@@ -327,7 +335,7 @@ int Engine::run(int model, int mode, const float *p0, float *pb, float *pr) {
   if(laplace) {
     KL_REQUIRE(mode == MODE_STEP || pr, KLRTM_EINVAL, "ISO needs the pr scratch volume");
     IsoArgs a;
-    fill_args(a, 2);
+    fill_args(a, 2, model);
     return launch_iso(ne, mode, p0, pb, vel, pr, a);
   }
   // first-derivative (TTI-alike) form: bgprtm/KernelCPU.cpp:93-119
@@ -336,7 +344,7 @@ int Engine::run(int model, int mode, const float *p0, float *pb, float *pr) {
   if((rc = scratch())) return rc;
   if(engine == KLRTM_ENGINE_CFD) return cfd_run(*this, model, mode, p0, pb, pr);
   IsoArgs a;
-  fill_args(a, 1);
+  fill_args(a, 1, model);
   if((rc = launch_grad(ne, model, p0, d_px, pr, d_pz, eps, del, pjx, pjy, a))) return rc;
   return launch_div(ne, mode, d_px, pr, d_pz, p0, pb, vel, a);
 }
@@ -431,7 +439,7 @@ int klrtm_kernel_laplacian(klrtm_kernel *kk, const float *in, float *out) {
   KL_REQUIRE(k->engine == KLRTM_ENGINE_FD, KLRTM_EINVAL, "laplacian() is an FD-engine operation");
   KL_REQUIRE(in != out, KLRTM_EINVAL, "laplacian() cannot run in place");
   IsoArgs a;
-  k->fill_args(a, 2);
+  k->fill_args(a, 2, KLRTM_ISO);
   return launch_iso(k->ne, MODE_LAP, in, nullptr, nullptr, out, a);
 }
 int klrtm_kernel_deriv1(klrtm_kernel *kk, int axis, const float *in, float *out, int iacc, int isign) {
@@ -449,7 +457,7 @@ int klrtm_kernel_deriv1(klrtm_kernel *kk, int axis, const float *in, float *out,
   }
   KL_REQUIRE(in != out, KLRTM_EINVAL, "FD derivative cannot run in place");
   IsoArgs a;
-  k->fill_args(a, 1);
+  k->fill_args(a, 1, KLRTM_ISO);
   return launch_deriv1(k->ne, axis, iacc, isign > 0 ? 0 : 1, in, out, k->vel, a);
 }
 int klrtm_kernel_set_zgrid(klrtm_kernel *kk, const float *zgrid) {
@@ -487,7 +495,7 @@ int klrtm_kernel_get_tile(klrtm_kernel *kk, int *tz, int *tx, int *ychunk) {
   Engine *k = reinterpret_cast<Engine *>(kk);
   KL_REQUIRE(k, KLRTM_EINVAL, "null engine");
   int a, b, c;
-  k->default_tile(k->ne, a, b, c);
+  k->default_tile(k->ne, false, false, a, b, c);  // as the Laplacian step runs
   if(tz) *tz = a;
   if(tx) *tx = b;
   if(ychunk) *ychunk = c;

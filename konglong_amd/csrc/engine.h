@@ -50,8 +50,8 @@ struct Engine {
   int ensure_comps(int comps);
   int clean();
   int set_boundary(const int *nbnd, float dt, float vmax);
-  void default_tile(int R, int &tz_out, int &tx_out, int &ychunk_out) const;
-  void fill_args(IsoArgs &a, int deriv_order);
+  void default_tile(int R, bool first_deriv, bool tti, int &tz_out, int &tx_out, int &ychunk_out) const;
+  void fill_args(IsoArgs &a, int deriv_order, int model);
   int check_model(int model);
   int scratch();
   int run(int model, int mode, const float *p0, float *pb, float *pr);
