@@ -44,6 +44,11 @@ template<int R, int MODE>
 __global__ void __launch_bounds__(512) iso_step_kernel(const float *__restrict__ u, float *__restrict__ w0,
                                                         const float *__restrict__ vel, float *__restrict__ pr,
                                                         const IsoArgs a) {
+  // Cache policy of the PML state.  Streamed, it leaves L2 to the volumes but splits the lines that two tiles share.
+  // Where a CU holds one workgroup the first wins on grids that fit L2 (FD16 96^3 20.4 -> 20.0 us, 128^3 27.3 -> 26.8;
+  // 160^3 to 400^3 the same within 0.5 %), where it holds two the second loses more (FD8 128^3 19.6 -> 22.7 us, 200^3
+  // 52 -> 70 us).
+  constexpr int QP = R >= 7 ? CPOL_NT : 0;
   extern __shared__ float s[];
   const int S = a.tz + 2 * R;
   const int nx = a.nx, ny = a.ny, nz = a.nz;
@@ -150,13 +155,13 @@ __global__ void __launch_bounds__(512) iso_step_kernel(const float *__restrict__
       N.hx0 = buf_ld(ru, ox0, 0), N.hx1 = buf_ld(ru, ox1, 0);
 #pragma unroll
       for(int r = 0; r < 2; r++) {
-        if(ZL) N.sz[r] = buf_ld(rq[0][r], zo == OOR ? OOR : zo + (uint32_t)y * zs, 0);
-        if(XL) N.sx[r] = buf_ld(rq[1][r], xo == OOR ? OOR : xo + (uint32_t)y * xs, 0);
+        if(ZL) N.sz[r] = buf_ld<QP>(rq[0][r], zo == OOR ? OOR : zo + (uint32_t)y * zs, 0);
+        if(XL) N.sx[r] = buf_ld<QP>(rq[1][r], xo == OOR ? OOR : xo + (uint32_t)y * xs, 0);
       }
       if(YL) {
         const uint32_t so = (yoff + (uint32_t)(y - jy0) * (uint32_t)nxz) * 4u;
 #pragma unroll
-        for(int r = 0; r < 2; r++) N.sy[r] = buf_ld(rq[2][r], oc, so);
+        for(int r = 0; r < 2; r++) N.sy[r] = buf_ld<QP>(rq[2][r], oc, so);
       }
     };
     // plane y: the loads of y+2 go out first; y's tile goes to LDS buffer y&1 (the barrier of y-1
@@ -210,21 +215,21 @@ __global__ void __launch_bounds__(512) iso_step_kernel(const float *__restrict__
         float Lz = round2(zc[0], zc[1], zc[2], L, s1, s2);
         L = zo != OOR ? Lz : L;
         const uint32_t o = zo == OOR ? OOR : zo + (uint32_t)y * zs;
-        buf_st(s1, rq[0][0], o, 0), buf_st(s2, rq[0][1], o, 0);
+        buf_st<QP>(s1, rq[0][0], o, 0), buf_st<QP>(s2, rq[0][1], o, 0);
       }
       if(XL) {
         float s1 = C.sx[0], s2 = C.sx[1];
         float Lx = round2(xc[0], xc[1], xc[2], L, s1, s2);
         L = xo != OOR ? Lx : L;
         const uint32_t ox = xo == OOR ? OOR : xo + (uint32_t)y * xs;
-        buf_st(s1, rq[1][0], ox, 0), buf_st(s2, rq[1][1], ox, 0);
+        buf_st<QP>(s1, rq[1][0], ox, 0), buf_st<QP>(s2, rq[1][1], ox, 0);
       }
       if(YL) {
         const cfloat *t = (const cfloat *)P.abc[fy][0] + 3 * (y - jy0);
         float s1 = C.sy[0], s2 = C.sy[1];
         L = round2(t[0], t[1], t[2], L, s1, s2);
         const uint32_t so = (yoff + (uint32_t)(y - jy0) * (uint32_t)nxz) * 4u;
-        buf_st(s1, rq[2][0], oc, so), buf_st(s2, rq[2][1], oc, so);
+        buf_st<QP>(s1, rq[2][0], oc, so), buf_st<QP>(s2, rq[2][1], oc, so);
       }
       if(MODE == MODE_STEP) {
         buf_st((ctr + ctr) - fmaf(-C.v, L, C.w), prs(w0, y), oc, 0);

@@ -123,11 +123,15 @@ constexpr uint32_t OOR = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
 }
+// (CPOL: cache policy, CPOL_NT streams past lines that other tiles still re-read from L2)
+constexpr int CPOL_NT = 2;
+template<int CPOL = 0>
 __device__ __forceinline__ float buf_ld(__amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, soff, 0));
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, soff, CPOL));
 }
+template<int CPOL = 0>
 __device__ __forceinline__ void buf_st(float v, __amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, voff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, voff, soff, CPOL);
 }
 // Workgroup barrier for LDS hand-off only: waits for this wave's LDS accesses
 // (lgkmcnt) but not for outstanding global loads, so prefetches issued before
