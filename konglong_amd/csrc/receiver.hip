@@ -697,9 +697,15 @@ int receiver_apply_at(Receiver &R, float *w0, const StepRef &ts, const float *ve
       continue;
     }
     const GatherTabs tabs = gather_tabs(R, g);
-    // the y factors of a few receivers are formed where they are used; many receivers reach a cell hundreds of
-    // times, where a factor read from memory beats two dependent loads
-    if(g.nr <= 4096) {
+    // The y factors (val*scaler)*ky are formed where they are used, which takes two dependent loads a term, or first by
+    // a launch of their own.  us with the one / the other form, scattered stations:
+    //   spread 10   20           100          300          1000         2000         4000         (terms a cell)
+    //   60^2        7.3 / 8.5    9.5 / 10.1  19.2 / 14.0  38.1 / 22.2  67.3 / 32.8  142 / 59      2 .. 440
+    //   128^2       5.8 / 7.4    7.0 / 8.7    9.5 / 10.0  16.9 / 13.6  20.9 / 15.1  32.9 / 20.7   0.5 .. 98
+    //   400^2      11.0 / 13.2  13.6 / 15.3  16.5 / 18.2  22.8 / 23.5  27.2 / 26.4  34.1 / 31.0   0.05 .. 10
+    // and with spread 5 even at 8 terms a cell (60^2, 300: 9.5 / 9.3), 12 (128^2, 2000: 10.4 / 10.3) and 2000 stations
+    // (400^2: 16.8 / 17.4, 4000: 21.1 / 20.2): the line lies at 12 terms a cell and at 2048 stations.
+    if(g.nr <= 2048 && (long)g.nr * g.lxmax * g.lymax <= 12L * cells) {
       hipLaunchKernelGGL(inject_gather_kernel<false>, dim3(div_up(cells, 64)), dim3(256), 0, stream(), a, tabs, tr, g.kz, w0,
                          vel);
     } else {

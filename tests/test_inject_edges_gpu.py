@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
 CASES = [  # ny, nx, stations, depths, mirror plane
     (40, 40, 1, 1, -1), (40, 40, 1, 1, 13), (30, 90, 7, 3, -1), (64, 71, 300, 2, 12), (90, 70, 5000, 1, -1),
     (43, 64, "grid1", 1, -1), (41, 65, "grid1", 1, 12), (45, 130, "grid2", 2, -1), (42, 30, "grid1", 1, 11),
+    # few and many stations on either side of 12 terms a cell (spread 6: 144 terms a station)
+    (40, 40, 90, 1, 12), (40, 40, 400, 1, -1), (50, 44, 2100, 2, 13), (190, 170, 2040, 1, -1), (190, 170, 2060, 1, -1),
 ]
 
 
