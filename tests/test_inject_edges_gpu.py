@@ -1,5 +1,5 @@
 """Injection and extraction at the edges of their workgroups against dense FP64 sums over the receivers' own taps:
-plane boxes below, at and past 64 columns and 4 rows, one station, few and many (> 4096) scattered stations, gridded
+plane boxes below, at and past 64 columns and 4 rows and past 65536 cells, one station, few and many (> 4096) scattered stations, gridded
 stations, several depths, and the ghost mirror.
 
 A cell's sum has at most a few hundred terms of one sign-mixed kernel product each: FP32 rounding of the terms and
@@ -18,6 +18,8 @@ CASES = [  # ny, nx, stations, depths, mirror plane
     (43, 64, "grid1", 1, -1), (41, 65, "grid1", 1, 12), (45, 130, "grid2", 2, -1), (42, 30, "grid1", 1, 11),
     # few and many stations on either side of 12 terms a cell (spread 6: 144 terms a station)
     (40, 40, 90, 1, 12), (40, 40, 400, 1, -1), (50, 44, 2100, 2, 13), (190, 170, 2040, 1, -1), (190, 170, 2060, 1, -1),
+    # a station at every cell of a box past 65536 cells (four plane rows a workgroup): 3 rows and 5 columns left over
+    (259, 261, "grid1", 1, -1), (259, 261, "grid1", 1, 12),
 ]
 
 
