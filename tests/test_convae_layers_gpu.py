@@ -1,7 +1,7 @@
 """Layers of the autoencoder near the edges of their tiles, and their weight gradients tap by tap.
 
 The upsampling layers are computed per output phase from the coarse grid in tiles of 2 x 8 x D cells, the
-output layer as sums over products with all taps in slabs of 8 rows: rough inputs and non-zero biases, so
+output layer in columns of 8 rows, cut along y for few blocks: rough inputs and non-zero biases, so
 that every tap, phase, halo and tile boundary carries weight, for one block and for odd counts.
 
 Bounds: the device and the reference round the same operands to BF16, but their FP32 summation orders
@@ -57,8 +57,9 @@ def test_every_cell_of_rough_blocks(klrtm, nb):
 
 @pytest.mark.parametrize("nb", [1, 5, 33])
 def test_weight_gradient_of_every_tap(klrtm, nb):
-    """The weight gradients tap by tap against torch autograd in FP32, for one block, and for numbers of
-    blocks whose tiles leave a remainder over the workgroups (256 of 64 tiles a block, 1024 of 8 slabs).
+    """The weight gradients tap by tap against torch autograd in FP32, for one block, and for numbers of blocks
+    whose tiles leave a remainder over the workgroups of the upsampling layers (64 tiles a block over 256, 8 over
+    128); the other layers have a workgroup for every task of these batches.
     Bound: each of K products carries two BF16 roundings (2^-9 each) and the layers before and behind add
     theirs; the eight layers together stay within 5e-2 as in the whole-layer comparison.  A tap taken from a
     neighbouring cell is uncorrelated with its reference."""
@@ -80,6 +81,40 @@ def test_weight_gradient_of_every_tap(klrtm, nb):
         print(f"[convae] layer {l}: largest tap error {max(e):.2e}", flush=True)
         worst = max(worst, max(e))
     assert worst < 5e-2
+
+
+@pytest.mark.parametrize("nb,active", [(67, (66,)), (67, (2, 66)), (131, (130,)), (131, (2, 130)), (259, (258,)),
+                                       (259, (2, 66, 130, 258))])
+def test_weight_gradient_of_blocks_past_the_first_round(klrtm, nb, active):
+    """Workgroups that take several tasks: 4 tiles a block of the 8^3 layers over 256 workgroups (a second task from
+    block 64 on), 8 slabs of the output layer and 4 of the input layer over 1024 (from blocks 128 and 256 on).  All
+    blocks but a few are zero, and so are their gradients as long as the biases are zero, so the batch's gradient
+    times nb is the sum of the few blocks' own, each from a call of one block, in which no workgroup takes a second
+    task.  Bound: the loss scale 1/nb moves the BF16 roundings of the gradients that pass the eight layers, 2^-9 each
+    and both sides rounded: 2 * sqrt(8) * 2^-9 = 1.1e-2, and as much again for the operands of the weight gradient.
+    A task that is lost or counted twice is a quarter or an eighth of one of at most four blocks: 3 % or more."""
+    print(f"[convae] weight gradients of {nb} blocks, all zero but {active}", flush=True)
+    h = C.c_void_p()
+    check(lib().klrtm_convae_create(C.byref(h), 24))
+    p = np.empty(lib().klrtm_convae_param_count(), np.float32)
+    check(lib().klrtm_convae_get_params(h.value, p.ctypes.data))
+    assert all(not b.any() for _, b in ref.split_params(p))
+    rng = np.random.default_rng(nb)
+    x = np.zeros((nb, 32, 32, 32), np.float32)
+    want = np.zeros(p.size)
+    for i in active:
+        x[i] = rng.standard_normal((32, 32, 32))
+    dx = DeviceArray.from_host(x)
+    g, loss = np.empty_like(p), C.c_float()
+    for i in active:
+        check(lib().klrtm_convae_loss_grad(h.value, dx.ptr + i * 131072, 1, g.ctypes.data, C.byref(loss)))
+        want += g
+    check(lib().klrtm_convae_loss_grad(h.value, dx.ptr, nb, g.ctypes.data, C.byref(loss)))
+    lib().klrtm_convae_destroy(h.value)
+    for l, ((w, _), (v, _)) in enumerate(zip(ref.split_params(g.astype(np.float64) * nb), ref.split_params(want))):
+        err = float(np.linalg.norm(w - v) / np.linalg.norm(v))
+        print(f"[convae] layer {l}: {err:.2e}", flush=True)
+        assert err < 2.2e-2
 
 
 def test_gradient_of_a_shifted_input(klrtm):
