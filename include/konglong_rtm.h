@@ -160,7 +160,8 @@ int klrtm_kernel_laplacian(klrtm_kernel *k, const float *in, float *out);
 int klrtm_kernel_deriv1(klrtm_kernel *k, int axis, const float *in, float *out, int iacc, int isign);
 /* tile shape of the stencil kernels: tz (z lanes), tx (x rows), ychunk (y planes per
  * block), tz*tx <= 512; 0 keeps the current value, ychunk < 0 returns to the default
- * chunking.  get_tile reports the shape the Laplacian step runs with.  On the compact (CFD)
+ * chunking.  get_tile reports the shape the Laplacian step runs with; the first-derivative passes
+ * (VTI, TTI, density) run at most 64 z lanes and 32 x rows of it.  On the compact (CFD)
  * engine tz is the number of lines per block of the x and y line passes (64, 128 or 256;
  * default 256) and tx, ychunk are ignored.  Used by the autotuner. */
 int klrtm_kernel_set_tile(klrtm_kernel *k, int tz, int tx, int ychunk);

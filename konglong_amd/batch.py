@@ -33,7 +33,7 @@ class Autotuner:
     TILES = ((64, 8), (64, 4), (32, 8), (128, 4))
     CFD_BLOCKS = (64, 128, 256)  # lanes per block of the compact engine's x/y line passes
     CFD_TIMERS = (b"cfd_step",)  # the step's span: its concurrent passes count once
-    TILES_FIRST_DERIV = TILES + ((16, 16),)  # the gradient/divergence kernels also take 16 x 16
+    TILES_FIRST_DERIV = TILES[:3] + ((16, 16),)  # the gradient/divergence kernels run at most 64 z lanes
     YCHUNKS = (0, 16, 32, 64)   # 0: the engine's default chunking
 
     def __init__(self, steps=4):

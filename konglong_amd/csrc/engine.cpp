@@ -271,6 +271,7 @@ int Engine::set_boundary(const int *nbnd, float dt_, float vmax_) {
 void Engine::default_tile(int R, bool first_deriv, bool tti, int &etz, int &etx, int &eyc) const {
   etz = tz > 0 ? tz : std::max(R, std::min(64, nz));
   etx = tx > 0 ? tx : std::max(R, 8);
+  if(first_deriv) etz = std::min(etz, TILE_Z), etx = std::min(etx, DERIV_TX);
   while(etz * etx > 512) etx = std::max(R, etx / 2);  // the stencil kernels are built for <= 512 threads
   eyc = ychunk;
   if(eyc > 0) return;

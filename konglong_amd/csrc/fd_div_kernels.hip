@@ -136,7 +136,7 @@ template<int R, int MODE, bool RHO>
 static int launch_div_rm(const float *px, const float *py, const float *pz, const float *w1, float *w0, const float *vel,
                          IsoArgs a) {
   LaunchTimer tm(MODE == MODE_STEP ? "fd_div_step" : "fd_div");
-  deriv_tile(a);
+  grid_of(a);
   size_t lds = 2 * sizeof(float) * ((size_t)a.tx * (TILE_Z + 2 * R) + (size_t)(a.tx + 2 * R) * TILE_Z);
   if(a.zc1) lds += sizeof(float) * (size_t)a.tz * (R + 1);
   hipLaunchKernelGGL((div_kernel<R, MODE, RHO>), dim3(a.nbz * a.nbx * a.nby), dim3(a.tz * a.tx), lds, stream(), px, py, pz, w1, w0, vel, a);

@@ -161,7 +161,7 @@ template<int R, int MODEL, bool RHO>
 static int launch_grad_rm(const float *u, float *px, float *py, float *pz, const float *eps, const float *del,
                           const float *pjx, const float *pjy, IsoArgs a) {
   LaunchTimer tm("fd_grad");
-  deriv_tile(a);
+  grid_of(a);
   size_t lds = sizeof(float) * (size_t)(R + 2) * (a.tx + 2 * R) * (TILE_Z + 2 * R);  // the ring of plane tiles
   if(a.zc1) lds += sizeof(float) * (size_t)a.tz * (R + 1);
   hipLaunchKernelGGL((grad_kernel<R, MODEL, RHO>), dim3(a.nbz * a.nbx * a.nby), dim3(a.tz * a.tx), lds, stream(), u, px, py, pz, eps, del, pjx, pjy, a);

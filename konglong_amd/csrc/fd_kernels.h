@@ -9,6 +9,11 @@ namespace klrtm {
 // density) and the CFD engine run it as MODE_KERNEL, which uses pr as scratch.
 enum { MODE_KERNEL = 0, MODE_STEP = 1, MODE_LAP = 2, MODE_PB = 3 };
 
+// Largest tile of the first-derivative passes: z lanes (the pitch of their LDS rows, a constant, so that the x
+// neighbours of a cell sit at immediate offsets; a runtime pitch took an address register and an add per x tap) and
+// x rows (R + 2 planes of 32 + 2R rows of 64 + 2R cells fill the LDS at R = 8).
+constexpr int TILE_Z = 64, DERIV_TX = 32;
+
 // Arguments of the y-streaming stencil kernels (passed by value).
 struct IsoArgs {
   int nx, ny, nz;

@@ -13,18 +13,6 @@ inline void grid_of(IsoArgs &a) {
 
 }  // namespace klrtm
 
-namespace klrtm {
-// LDS row pitch of the z dimension of a tile: a constant, so that the x neighbours of a cell sit at immediate
-// offsets (a runtime pitch took an address register and an add per x tap).
-constexpr int TILE_Z = 64;
-
-// tile and grid of a first-derivative pass: tz within the LDS pitch, tx within the LDS of tall tiles
-inline void deriv_tile(IsoArgs &a) {
-  a.tz = a.tz < TILE_Z ? a.tz : TILE_Z, a.tx = a.tx < 32 ? a.tx : 32;
-  grid_of(a);
-}
-}  // namespace klrtm
-
 #ifdef __HIPCC__
 namespace klrtm {
 

@@ -3,6 +3,7 @@ the fastest, for orders 8, 10, 12 and 16 and grids of 48 to 400 planes.  (3 plan
 long as 7, and 3 planes at 96^3 1.41 times as long as 10.)"""
 import pytest
 
+from konglong_amd.batch import Autotuner
 from konglong_amd.kernel import KernelCPU
 
 BEST = {  # (ny, nx, nz): chunks for orders 8, 10, 12 and for 16
@@ -39,3 +40,10 @@ def test_chunk_lies_in_the_grid(ny, tile):
     assert k.get_tile()[2] == 9
     k.set_tile(0, 0, -1)
     assert 1 <= k.get_tile()[2] <= ny
+
+
+def test_autotuner_times_no_tile_twice():
+    """The first-derivative passes run at most 64 z lanes, so a wider candidate is another one again."""
+    seen = [(min(tz, 64), min(tx, 32)) for tz, tx in Autotuner.TILES_FIRST_DERIV]
+    assert len(set(seen)) == len(seen)
+    assert all(t in Autotuner.TILES_FIRST_DERIV for t in ((64, 8), (64, 4), (32, 8), (16, 16)))
