@@ -486,6 +486,7 @@ int klrtm_kernel_set_tile(klrtm_kernel *kk, int tz, int tx, int ychunk) {
   if(tx > 0) KL_REQUIRE(tx >= R, KLRTM_EINVAL, "tile tx must be >= stencil radius %d", R);
   int ntz = tz > 0 ? tz : k->tz, ntx = tx > 0 ? tx : k->tx;
   if(ntz > 0 && ntx > 0) KL_REQUIRE(ntz * ntx <= 512, KLRTM_EINVAL, "tile tz*tx must be <= 512");
+  else if(ntz > 0) KL_REQUIRE(ntz * R <= 512, KLRTM_EINVAL, "tile tz %d leaves no room for %d x rows in 512 threads", ntz, R);
   if(tz > 0) k->tz = tz;
   if(tx > 0) k->tx = tx;
   if(ychunk > 0) k->ychunk = ychunk;

@@ -42,6 +42,19 @@ def test_chunk_lies_in_the_grid(ny, tile):
     assert 1 <= k.get_tile()[2] <= ny
 
 
+def test_tile_without_room_is_refused():
+    """128 z lanes leave 4 x rows in 512 threads, the radius of FD16 is 8: no x tile fits, and looking for one by
+    halving never ended."""
+    k = KernelCPU(64, 64, 256, 10.0, 10.0, 10.0, order=16)
+    before = k.get_tile()
+    with pytest.raises(Exception, match="no room"):
+        k.set_tile(128)
+    assert k.get_tile() == before
+    k = KernelCPU(64, 64, 256, 10.0, 10.0, 10.0, order=8)
+    k.set_tile(128)
+    assert k.get_tile()[:2] == (128, 4)
+
+
 def test_autotuner_times_no_tile_twice():
     """The first-derivative passes run at most 64 z lanes, so a wider candidate is another one again."""
     seen = [(min(tz, 64), min(tx, 32)) for tz, tx in Autotuner.TILES_FIRST_DERIV]
