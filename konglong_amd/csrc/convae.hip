@@ -1007,7 +1007,7 @@ int cae_reserve(CaeWork &w, int nb, bool train) {
   for(int l = 0; l < CAE_LAYERS; l++) {
     const size_t no = (size_t)nb * kCout[l] * ((size_t)kDout[l] * kDout[l] * kDout[l]);
     KL_HIP(hipMalloc(&w.a[l], no * 4));
-    if(train) KL_HIP(hipMalloc(&w.z[l], no * 4));
+    if(train && kGelu[l]) KL_HIP(hipMalloc(&w.z[l], no * 4));  // (read by the gradient through the activation only)
     // gradient buffers: this layer's output gradient, its input gradient, and for upsampling layers
     // the input gradient on the fine grid
     const size_t ni = (size_t)nb * kCin[l] * ((size_t)kDin[l] * kDin[l] * kDin[l]);
