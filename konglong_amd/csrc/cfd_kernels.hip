@@ -339,7 +339,7 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
     for(int k = 0; k < 10; k++) X[k] = X[k + 1];
     X[10] = v;
   };
-  auto eliminate = [&](int i, float acc) __attribute__((always_inline)) {  // (i >= 5: all four terms)
+  auto eliminate = [&](int i, float acc) __attribute__((always_inline)) {
     if(i >= 4) acc = acc - Lw[(i - 4) * 4 + 3] * B3;
     if(i >= 3) acc = acc - Lw[(i - 3) * 4 + 2] * B2;
     if(i >= 2) acc = acc - Lw[(i - 2) * 4 + 1] * B1;
@@ -359,7 +359,7 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
   auto interior = [&]() {
     return a55 * (X[6] - X[4]) + a56 * (X[7] - X[3]) + a57 * (X[8] - X[2]) + a58 * (X[9] - X[1]) + a59 * (X[10] - X[0]);
   };
-  auto eliminate4 = [&](int i, float acc) __attribute__((always_inline)) {
+  auto eliminate4 = [&](int i, float acc) __attribute__((always_inline)) {  // i >= 5: all four terms
     acc = acc - Lw[(i - 4) * 4 + 3] * B3;
     acc = acc - Lw[(i - 3) * 4 + 2] * B2;
     acc = acc - Lw[(i - 2) * 4 + 1] * B1;
@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(256) cfd_line_kernel(const float *in, float *t
 // transposed tiles, so every global access of the pass is coalesced.
 // Interior chunks are fully unrolled: the 11-sample window lives in renamed
 // registers and the plan rows and samples of half a chunk are read before its
-// solves (121^3: 76 -> 70 us).
+// solves (121x97x113: 81 -> 73 us; 400^3: 430 us either way, bound by memory).
 // Global memory is reached through per-wave buffer resources; tile elements
 // beyond the line or the last line get an out-of-range offset, so their loads
 // return 0 and their stores are dropped, and no access needs a branch.

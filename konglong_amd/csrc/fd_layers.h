@@ -6,19 +6,19 @@
 //
 // Both stream along y like the Laplacian step: a block owns a (TZ x TX) tile of the (z,x) plane, keeps the
 // 2R+1 y-neighbours of its column in registers and stages the plane's z/x halos in LDS.  They are bound by
-// HBM (gradient 12-28 bytes in and 12 out per cell, divergence 24 in and 4 out, plus 8 bytes per damped cell
+// HBM (gradient 8-24 bytes in and 12 out per cell, divergence 24-28 in and 4 out, plus 8 bytes per damped cell
 // and component), which takes memory requests in flight and lines read once, not arithmetic.  The first form
 // copied one prefetched plane between registers and read the PML state where it was used: two thirds of the
 // wave cycles waited for loads.  Here
 //  * the loads of plane y+1, PML state included, go out unconditionally before plane y is computed, into the
 //    other of two register sets;
 //  * the gradient loads halos R planes ahead, with the own column's sample of the same plane, when neighbour
-//    blocks load the same lines (R+2 plane tiles in LDS; 3.5 -> 3.1 GB fetched in the interior of a TTI step);
+//    blocks load the same lines (R+2 plane tiles in LDS);
 //  * LDS pitches are constants (an address register and an add per x tap otherwise), blocks that touch no
 //    layer run code without any, and nothing is loaded or stored with the streaming cache policy: a tile's
-//    rows end inside 128-byte lines that its z neighbour reads too (VTI 301x277x333: 0.76 -> 0.61 ms a step).
-// MI355X, a whole step before and after: TTI FD16 600x600x400 5.46 -> 3.60 ms (15.7 GB needed for two steps:
-// 2.2 TB/s), TTI FD16 300^3 1.39 -> 0.78 ms, VTI FD8 301x277x333 0.96 -> 0.61 ms.
+//    rows end inside 128-byte lines that its z neighbour reads too (VTI 301x277x333: 20 % less time a step).
+// MI355X, a whole step before and after: TTI FD16 600x600x400 5.45 -> 3.73 ms (14.4 GB moved at 3.8 TB/s, 7.8 GB
+// needed), TTI FD16 300^3 1.19 -> 0.69 ms, VTI FD8 301x277x333 0.96 -> 0.62 ms.
 #pragma once
 #include "fd_tile.h"
 #include "stencil_common.h"
