@@ -346,6 +346,10 @@ int Engine::run(int model, int mode, const float *p0, float *pb, float *pr) {
   if(engine == KLRTM_ENGINE_CFD) return cfd_run(*this, model, mode, p0, pb, pr);
   IsoArgs a;
   fill_args(a, 1, model);
+  if(ny == 1) {
+    if((rc = launch_grad_plane(ne, model, p0, d_px, d_pz, eps, del, pjx, a))) return rc;
+    return launch_div_plane(ne, mode, d_px, d_pz, p0, pb, vel, a);
+  }
   if((rc = launch_grad(ne, model, p0, d_px, pr, d_pz, eps, del, pjx, pjy, a))) return rc;
   return launch_div(ne, mode, d_px, pr, d_pz, p0, pb, vel, a);
 }

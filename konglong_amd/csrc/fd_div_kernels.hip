@@ -32,14 +32,12 @@ __global__ void __launch_bounds__(512) div_kernel(const float *__restrict__ px, 
   const int tile = TX * SZ + (TX + 2 * R) * SX;  // TX rows of the first tile, TX+2R rows of the second
   const LayerSlots sl = layer_slots(c, a);
   const LayerOps L(a, sl, 1, c);
-  const bool do_y = ny > 1;
-  const float *pyl = do_y ? py : px;  // 2D: loaded, not used
   auto prs = [&](const float *base, int y) { return buf_rsrc(base + (size_t)y * nxz, pbytes); };
   float q[2 * R + 1];
 #pragma unroll
   for(int k = 0; k < 2 * R; k++) {
     const int yy = c.y0 - R + k;
-    q[k] = (do_y && c.act && yy >= 0 && yy < ny) ? py[(size_t)yy * nxz + c.col] : 0.f;
+    q[k] = (c.act && yy >= 0 && yy < ny) ? py[(size_t)yy * nxz + c.col] : 0.f;
   }
   float *zrow0 = s + c.tx * SZ + c.tz + R;                 // LDS tiles of even planes
   float *xrow0 = s + TX * SZ + (c.tx + R) * SX + c.tz;
@@ -61,7 +59,7 @@ __global__ void __launch_bounds__(512) div_kernel(const float *__restrict__ px, 
     auto fetch = [&](Plane &N, int y) __attribute__((always_inline)) {
       const __amdgpu_buffer_rsrc_t rz = prs(pz, y), rx = prs(px, y);
       const size_t pl = (size_t)y * nxz;
-      N.qa = at_ld(pyl + (size_t)min(y + R, ny - 1) * nxz, L.col);
+      N.qa = at_ld(py + (size_t)min(y + R, ny - 1) * nxz, L.col);
       N.cz = buf_ld(rz, o.c, 0), N.hz0 = buf_ld(rz, o.z0, 0), N.hz1 = buf_ld(rz, o.z1, 0);
       N.cx = buf_ld(rx, o.c, 0), N.hx0 = buf_ld(rx, o.x0, 0), N.hx1 = buf_ld(rx, o.x1, 0);
       N.w = at_ld(w0 + pl, L.col);
@@ -102,7 +100,7 @@ __global__ void __launch_bounds__(512) div_kernel(const float *__restrict__ px, 
 #pragma unroll
         for(int m = 1; m <= R; m++) dzv = fmaf(a.cz[m], zrow[m], dzv);
       }
-      float dyv = 0.f;  // (2D: zero)
+      float dyv = 0.f;
 #pragma unroll
       for(int m = 1; m <= R; m++) {
         dyv = fmaf(-a.cy[m], q[R - m], dyv);

@@ -28,8 +28,9 @@ __global__ void __launch_bounds__(512) grad_kernel(const float *__restrict__ u, 
   const TileOffsets o = tile_offsets<R>(c, a);
   const LayerSlots sl = layer_slots(c, a);
   const LayerOps L(a, sl, 0, c);
-  const bool do_y = ny > 1, st_y = c.act && do_y;
-  const float *pjyl = do_y ? pjy : pjx;  // 2D: loaded, not used
+  // (ny > 1: a 2D grid has kernels of its own.  Asked for again because a branch of its own keeps gy's last products in
+  // its block, and with them what the compiler contracts there: the bits of the step)
+  const bool st_y = c.act && ny > 1;
   auto prs = [&](const float *base, int y) { return buf_rsrc(base + (size_t)y * nxz, pbytes); };
   float q[2 * R + 1];
 #pragma unroll
@@ -88,7 +89,7 @@ __global__ void __launch_bounds__(512) grad_kernel(const float *__restrict__ u, 
       }
       if(MODEL == KLRTM_TTI) {
         N.ax = at_ld(pjx + pl, L.col);
-        N.ay = at_ld(pjyl + pl, L.col);
+        N.ay = at_ld(pjy + pl, L.col);
       }
       if(RHO) N.rho = at_ld(a.rho + pl, L.col);
       N.hz0 = buf_ld(ru, o.z0, 0), N.hz1 = buf_ld(ru, o.z1, 0);
@@ -126,7 +127,7 @@ __global__ void __launch_bounds__(512) grad_kernel(const float *__restrict__ u, 
         gx = fmaf(-a.cx[m], srow[-m * S], gx);
         gx = fmaf(a.cx[m], srow[m * S], gx);
       }
-      float gy = 0.f;  // (2D: every y neighbour is zero)
+      float gy = 0.f;
 #pragma unroll
       for(int m = 1; m <= R; m++) {
         gy = fmaf(-a.cy[m], q[R - m], gy);
@@ -141,7 +142,7 @@ __global__ void __launch_bounds__(512) grad_kernel(const float *__restrict__ u, 
         gz /= C.rho;
       }
       if(MODEL == KLRTM_VTI) scalar_vti(C.e, C.d, gx, gy, gz);
-      else if(MODEL == KLRTM_TTI) scalar_tti(C.e, C.d, C.ax, do_y ? C.ay : 0.f, gx, gy, gz);
+      else if(MODEL == KLRTM_TTI) scalar_tti(C.e, C.d, C.ax, C.ay, gx, gy, gz);
       if(c.act) {
         const size_t pl = (size_t)y * nxz;
         at_st(px + pl, L.col, gx);

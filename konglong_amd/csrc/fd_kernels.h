@@ -36,6 +36,11 @@ int launch_grad(int R, int model, const float *u, float *px, float *py, float *p
                 const float *pjx, const float *pjy, const IsoArgs &a);
 int launch_div(int R, int mode, const float *px, const float *py, const float *pz, const float *w1, float *w0,
                const float *vel, const IsoArgs &a);
+// the same passes on a 2D grid (ny 1)
+int launch_grad_plane(int R, int model, const float *u, float *px, float *pz, const float *eps, const float *del,
+                      const float *pjx, const IsoArgs &a);
+int launch_div_plane(int R, int mode, const float *px, const float *pz, const float *w1, float *w0, const float *vel,
+                     const IsoArgs &a);
 int launch_deriv1(int R, int axis, int iacc, int round, const float *in, float *out, const float *vel, const IsoArgs &a);
 int launch_vel2(float *v, size_t n, float dt);
 int launch_update2nd(float *w0, const float *w1, size_t n);

@@ -2,7 +2,7 @@
 
 The first-derivative passes work on 64 x 8 tiles (z lanes x x rows) with a ring of R+2 plane tiles, and drop the
 PML code in blocks that touch no layer: grids just below, at and past a tile, fewer planes than the stencil's
-radius, 2D, layers on some faces only and without the cross axes.  Both sides run FP32 in different
+radius, 2D (kernels of its own), layers on some faces only and without the cross axes.  Both sides run FP32 in different
 association: a step adds at most about 6 roundings of 6e-8 of the field per cell, which four leapfrog steps
 (errors grow with the square of the step count, 10 step errors in all) turn into 4e-6 relative."""
 import numpy as np
@@ -29,6 +29,12 @@ CASES = [
     ((37, 40, 10), 8, VTI, (6, 7, 5, 8, 3, 4), True, (4, 128, 7)),
     ((6, 9, 65), 8, ISO, (2, 2, 2, 2, 10, 10), True, None),
     ((70, 8, 129), 16, ISO, (0, 0, 0, 20, 0, 33), True, (64, 8, 1)),
+    # 2D: one layer, no layer, no cross axes, tiles of other shapes, several tiles with a rest on both axes
+    ((1, 70, 129), 16, VTI, (0, 9, 0, 0, 20, 0), False, None),
+    ((1, 64, 64), 12, VTI, (0, 0, 0, 0, 0, 0), True, None),
+    ((1, 9, 20), 8, TTI, (2, 3, 0, 0, 5, 5), True, (16, 16, 5)),
+    ((1, 41, 300), 14, TTI, (8, 8, 0, 0, 0, 31), True, (32, 16, 1)),
+    ((1, 130, 33), 10, VTI, (20, 60, 0, 0, 3, 4), True, (8, 64, 1)),
 ]
 
 
