@@ -38,10 +38,33 @@ template<int W> __device__ __forceinline__ C16Chunk c16_chunk(const uint16_t *co
   else k.j0 = lead + (c - 1) * W, k.n = k.j0 < nxz ? (unsigned)min((size_t)W, nxz - k.j0) : 0u;
   return k;
 }
-static unsigned c16_blocks(size_t nxz, int W) { return (unsigned)(((nxz + W - 1) / W + 1 + 255) / 256); }
 constexpr int C16_ENC = 8, C16_DEC = 4;  // (a wave's stores are contiguous: 16 bytes a lane on either side)
-constexpr int C16_DEC_U = 4;             // decode chunks per thread
-constexpr int C16_GRID_Y = 65535;  // slices per launch
+constexpr int C16_GRID_Y = 65535;        // slices per launch
+// Threads of a workgroup: chunks of one slice (blockIdx.y), or where a slice has at most 128 chunks, of as many
+// slices as fit 256 threads (60 000 slices of 32 samples: encode with its maxima 86 -> 35 us, decode 42 -> 7).
+struct C16Map {
+  unsigned cps, spb;  // chunks of a slice; slices of a workgroup (1: the slice has workgroups of its own)
+  int ny;
+};
+static C16Map c16_map(size_t nxz, int W, int ny) {
+  C16Map m;
+  const size_t cps = (nxz + W - 1) / W + 1;
+  m.cps = (unsigned)std::min<size_t>(cps, 256), m.spb = cps <= 128 ? 256 / m.cps : 1, m.ny = ny;
+  return m;
+}
+// grid of a launch over ny slices with U chunks a thread
+static dim3 c16_grid(const C16Map &m, size_t nxz, int W, int U, int ny) {
+  if(m.spb > 1) return dim3((unsigned)div_up(ny, m.spb));
+  return dim3((unsigned)(((nxz + W - 1) / W + 1 + 256 * U - 1) / (256 * U)), (unsigned)ny);
+}
+// slice and first chunk of a thread (iy >= m.ny: nothing); the next of its U chunks are 256 on
+__device__ __forceinline__ void c16_place(const C16Map &m, int U, int &iy, size_t &c) {
+  iy = blockIdx.y, c = (size_t)blockIdx.x * U * 256 + threadIdx.x;
+  if(m.spb == 1) return;
+  const unsigned sl = threadIdx.x / m.cps;
+  iy = sl < m.spb ? (int)(blockIdx.x * m.spb + sl) : m.ny;
+  c = threadIdx.x - sl * m.cps;
+}
 
 // per-slice max |x| (bgprtm/WaveFieldCompress.cpp:149-153); non-negative FP32
 // compare like their bit patterns, so atomicMax on the bits is exact and
@@ -77,9 +100,11 @@ __global__ void __launch_bounds__(256) slice_absmax_kernel(const float *__restri
 // Bound by HBM: 4 bytes in, 2 out per sample.  One sample per thread, 64-bit index division and divergent code
 // ranges ran at 1.8 TB/s (400^3: 217 us); eight samples per thread with 16-byte accesses take 66 us (5.9 TB/s).
 __global__ void __launch_bounds__(256) c16_encode_kernel(const float *__restrict__ in, uint16_t *__restrict__ out,
-                                                         const unsigned *__restrict__ smax, size_t nxz) {
-  const int iy = blockIdx.y;
-  const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
+                                                         const unsigned *__restrict__ smax, size_t nxz, const C16Map m) {
+  int iy;
+  size_t c;
+  c16_place(m, 1, iy, c);
+  if(iy >= m.ny) return;
   uint16_t *pout = out + (size_t)iy * (nxz + 2);
   const C16Chunk k = c16_chunk<C16_ENC>(pout + 2, nxz, c);
   const float vmax = __uint_as_float(smax[iy]);
@@ -105,22 +130,27 @@ __global__ void __launch_bounds__(256) c16_encode_kernel(const float *__restrict
 // 2 bytes in, 4 out per sample.  The edge taper's factors (one per axis; the low and high edges do not overlap) come
 // from a table in LDS that holds 1 past the taper: nearly every wave reaches a tapered z, and reading the factors
 // from the arguments under a branch cost more than the volume (400^3: 277 us, now about 85).
+template<int U>
 __global__ void __launch_bounds__(256) c16_decode_kernel(const uint16_t *__restrict__ in, float *__restrict__ out, int nx,
-                                                         int ny, int nz, int y0, const EdgeTaper T) {
+                                                         int ny, int nz, int y0, const EdgeTaper T, const C16Map m) {
   __shared__ float wt[21], wzt[11];
   if(threadIdx.x < 20) wt[threadIdx.x] = T.wt[threadIdx.x];
   if(threadIdx.x < 10) wzt[threadIdx.x] = T.wzt[threadIdx.x];
   if(threadIdx.x == 0) wt[20] = wzt[10] = 1.f;
   __syncthreads();
   const size_t nxz = (size_t)nx * nz;
-  const int iy = y0 + (int)blockIdx.y;
+  int iy;
+  size_t c0;
+  c16_place(m, U, iy, c0);
+  if(iy >= m.ny) return;
+  iy += y0;
   const uint16_t *pin = in + (size_t)iy * (nxz + 2);
   const float scale = __uint_as_float((unsigned)pin[0] | ((unsigned)pin[1] << 16));
   const bool on = scale > 1e-25f;
   const float fy = ny > 40 ? wt[min(min(iy, ny - 1 - iy), 20)] : 1.f;
 #pragma unroll
-  for(int u = 0; u < C16_DEC_U; u++) {
-    const C16Chunk k = c16_chunk<C16_DEC>(pin + 2, nxz, ((size_t)blockIdx.x * C16_DEC_U + u) * 256 + threadIdx.x);
+  for(int u = 0; u < U; u++) {
+    const C16Chunk k = c16_chunk<C16_DEC>(pin + 2, nxz, c0 + u * 256);
     if(k.n == 0) continue;  // past the end, or an empty first chunk
     float *pout = out + (size_t)iy * nxz + k.j0;
     int ix = nxz >> 32 ? (int)(k.j0 / nz) : (int)((unsigned)k.j0 / (unsigned)nz), iz = (int)(k.j0 - (size_t)ix * nz);
@@ -163,9 +193,12 @@ int c16_slice_max(const float *in, int nx, int ny, int nz, unsigned *smax) {
 
 static int c16_encode_slices(const float *in, uint16_t *out, int nx, int ny, int nz, const unsigned *smax) {
   const size_t nxz = (size_t)nx * nz;
-  for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y)
-    hipLaunchKernelGGL(c16_encode_kernel, dim3(c16_blocks(nxz, C16_ENC), std::min(ny - y0, C16_GRID_Y)), dim3(256), 0, stream(),
-                       in + (size_t)y0 * nxz, out + (size_t)y0 * (nxz + 2), smax + y0, nxz);
+  for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y) {
+    const int n = std::min(ny - y0, C16_GRID_Y);
+    const C16Map m = c16_map(nxz, C16_ENC, n);
+    hipLaunchKernelGGL(c16_encode_kernel, c16_grid(m, nxz, C16_ENC, 1, n), dim3(256), 0, stream(), in + (size_t)y0 * nxz,
+                       out + (size_t)y0 * (nxz + 2), smax + y0, nxz, m);
+  }
   return check_launch("c16_encode_kernel");
 }
 
@@ -178,9 +211,18 @@ int c16_encode(const float *in, uint16_t *out, int nx, int ny, int nz, unsigned 
 
 int c16_decode(const uint16_t *in, float *out, int nx, int ny, int nz) {
   LaunchTimer tm("c16_decode");
-  for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y)
-    hipLaunchKernelGGL(c16_decode_kernel, dim3(div_up(c16_blocks((size_t)nx * nz, C16_DEC), C16_DEC_U), std::min(ny - y0, C16_GRID_Y)), dim3(256), 0,
-                       stream(), in, out, nx, ny, nz, y0, make_edge_taper());
+  const size_t nxz = (size_t)nx * nz;
+  for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y) {
+    const int n = std::min(ny - y0, C16_GRID_Y);
+    const C16Map m = c16_map(nxz, C16_DEC, n);
+    // four chunks a thread share the tapers' table and the slice's scale, where that leaves two workgroups a CU
+    const dim3 four = c16_grid(m, nxz, C16_DEC, 4, n);
+    if(m.spb == 1 && (size_t)four.x * four.y >= 512)
+      hipLaunchKernelGGL(c16_decode_kernel<4>, four, dim3(256), 0, stream(), in, out, nx, ny, nz, y0, make_edge_taper(), m);
+    else
+      hipLaunchKernelGGL(c16_decode_kernel<1>, c16_grid(m, nxz, C16_DEC, 1, n), dim3(256), 0, stream(), in, out, nx, ny, nz,
+                         y0, make_edge_taper(), m);
+  }
   return check_launch("c16_decode_kernel");
 }
 

@@ -20,7 +20,10 @@ class At:
 
 @pytest.mark.parametrize("shape,fo,co", [((1, 1, 1), 0, 0), ((4, 1, 3), 0, 0), ((5, 3, 5), 4, 2), ((9, 7, 13), 8, 6),
                                          ((45, 43, 21), 4, 10), ((3, 130, 127), 0, 0), ((2, 256, 64), 12, 14),
-                                         ((42, 41, 200), 0, 4)])
+                                         ((42, 41, 200), 0, 4),
+                                         # several slices a workgroup: up to 1016 samples encoding, 508 decoding
+                                         ((300, 4, 8), 0, 0), ((41, 10, 16), 4, 2), ((70, 1, 31), 0, 6), ((3, 127, 8), 0, 0),
+                                         ((3, 113, 9), 8, 10), ((9, 127, 4), 0, 2), ((9, 509, 1), 4, 0), ((5, 1, 1), 0, 14)])
 def test_chunks_bit_exact(klrtm, shape, fo, co):
     print(f"[c16] {shape}, volume at +{fo}, codes at +{co} bytes", flush=True)
     ny, nx, nz = shape
