@@ -58,9 +58,10 @@ static dim3 c16_grid(const C16Map &m, size_t nxz, int W, int U, int ny) {
   return dim3((unsigned)(((nxz + W - 1) / W + 1 + 256 * U - 1) / (256 * U)), (unsigned)ny);
 }
 // slice and first chunk of a thread (iy >= m.ny: nothing); the next of its U chunks are 256 on
-__device__ __forceinline__ void c16_place(const C16Map &m, int U, int &iy, size_t &c) {
+template<int U, bool SHARED>
+__device__ __forceinline__ void c16_place(const C16Map &m, int &iy, size_t &c) {
   iy = blockIdx.y, c = (size_t)blockIdx.x * U * 256 + threadIdx.x;
-  if(m.spb == 1) return;
+  if(!SHARED) return;
   const unsigned sl = threadIdx.x / m.cps;
   iy = sl < m.spb ? (int)(blockIdx.x * m.spb + sl) : m.ny;
   c = threadIdx.x - sl * m.cps;
@@ -99,12 +100,13 @@ __global__ void __launch_bounds__(256) slice_absmax_kernel(const float *__restri
 
 // Bound by HBM: 4 bytes in, 2 out per sample.  One sample per thread, 64-bit index division and divergent code
 // ranges ran at 1.8 TB/s (400^3: 217 us); eight samples per thread with 16-byte accesses take 66 us (5.9 TB/s).
+template<bool SHARED>
 __global__ void __launch_bounds__(256) c16_encode_kernel(const float *__restrict__ in, uint16_t *__restrict__ out,
                                                          const unsigned *__restrict__ smax, size_t nxz, const C16Map m) {
   int iy;
   size_t c;
-  c16_place(m, 1, iy, c);
-  if(iy >= m.ny) return;
+  c16_place<1, SHARED>(m, iy, c);
+  if(SHARED && iy >= m.ny) return;
   uint16_t *pout = out + (size_t)iy * (nxz + 2);
   const C16Chunk k = c16_chunk<C16_ENC>(pout + 2, nxz, c);
   const float vmax = __uint_as_float(smax[iy]);
@@ -130,7 +132,7 @@ __global__ void __launch_bounds__(256) c16_encode_kernel(const float *__restrict
 // 2 bytes in, 4 out per sample.  The edge taper's factors (one per axis; the low and high edges do not overlap) come
 // from a table in LDS that holds 1 past the taper: nearly every wave reaches a tapered z, and reading the factors
 // from the arguments under a branch cost more than the volume (400^3: 277 us, now about 85).
-template<int U>
+template<int U, bool SHARED>
 __global__ void __launch_bounds__(256) c16_decode_kernel(const uint16_t *__restrict__ in, float *__restrict__ out, int nx,
                                                          int ny, int nz, int y0, const EdgeTaper T, const C16Map m) {
   __shared__ float wt[21], wzt[11];
@@ -141,8 +143,8 @@ __global__ void __launch_bounds__(256) c16_decode_kernel(const uint16_t *__restr
   const size_t nxz = (size_t)nx * nz;
   int iy;
   size_t c0;
-  c16_place(m, U, iy, c0);
-  if(iy >= m.ny) return;
+  c16_place<U, SHARED>(m, iy, c0);
+  if(SHARED && iy >= m.ny) return;
   iy += y0;
   const uint16_t *pin = in + (size_t)iy * (nxz + 2);
   const float scale = __uint_as_float((unsigned)pin[0] | ((unsigned)pin[1] << 16));
@@ -196,8 +198,13 @@ static int c16_encode_slices(const float *in, uint16_t *out, int nx, int ny, int
   for(int y0 = 0; y0 < ny; y0 += C16_GRID_Y) {
     const int n = std::min(ny - y0, C16_GRID_Y);
     const C16Map m = c16_map(nxz, C16_ENC, n);
-    hipLaunchKernelGGL(c16_encode_kernel, c16_grid(m, nxz, C16_ENC, 1, n), dim3(256), 0, stream(), in + (size_t)y0 * nxz,
-                       out + (size_t)y0 * (nxz + 2), smax + y0, nxz, m);
+    const dim3 grid = c16_grid(m, nxz, C16_ENC, 1, n);
+    const float *pin = in + (size_t)y0 * nxz;
+    uint16_t *pout = out + (size_t)y0 * (nxz + 2);
+    if(m.spb > 1)
+      hipLaunchKernelGGL(c16_encode_kernel<true>, grid, dim3(256), 0, stream(), pin, pout, smax + y0, nxz, m);
+    else
+      hipLaunchKernelGGL(c16_encode_kernel<false>, grid, dim3(256), 0, stream(), pin, pout, smax + y0, nxz, m);
   }
   return check_launch("c16_encode_kernel");
 }
@@ -217,11 +224,14 @@ int c16_decode(const uint16_t *in, float *out, int nx, int ny, int nz) {
     const C16Map m = c16_map(nxz, C16_DEC, n);
     // four chunks a thread share the tapers' table and the slice's scale, where that leaves two workgroups a CU
     const dim3 four = c16_grid(m, nxz, C16_DEC, 4, n);
-    if(m.spb == 1 && (size_t)four.x * four.y >= 512)
-      hipLaunchKernelGGL(c16_decode_kernel<4>, four, dim3(256), 0, stream(), in, out, nx, ny, nz, y0, make_edge_taper(), m);
+    const dim3 one = c16_grid(m, nxz, C16_DEC, 1, n);
+    const EdgeTaper T = make_edge_taper();
+    if(m.spb > 1)
+      hipLaunchKernelGGL((c16_decode_kernel<1, true>), one, dim3(256), 0, stream(), in, out, nx, ny, nz, y0, T, m);
+    else if((size_t)four.x * four.y >= 512)
+      hipLaunchKernelGGL((c16_decode_kernel<4, false>), four, dim3(256), 0, stream(), in, out, nx, ny, nz, y0, T, m);
     else
-      hipLaunchKernelGGL(c16_decode_kernel<1>, c16_grid(m, nxz, C16_DEC, 1, n), dim3(256), 0, stream(), in, out, nx, ny, nz,
-                         y0, make_edge_taper(), m);
+      hipLaunchKernelGGL((c16_decode_kernel<1, false>), one, dim3(256), 0, stream(), in, out, nx, ny, nz, y0, T, m);
   }
   return check_launch("c16_decode_kernel");
 }
