@@ -261,8 +261,8 @@ int Engine::set_boundary(const int *nbnd, float dt_, float vmax_) {
 // block's halo planes and first loads cost, and w the planes' time of waiting per plane of a round of resident
 // blocks, which only a second resident block fills.  Where a CU holds two workgroups of 8 waves (kernels of <= 128
 // VGPRs: the Laplacian up to FD12, both first-derivative passes up to FD10; one of the two up to FD12, and up to FD16
-// in VTI) h is R / 2 and w 1.5 (one pass of two: 0.5), and past two blocks a CU the blocks partly even out by
-// themselves (x, the mean, has its share beside k); where it holds one, h is 10 and w 0.1.
+// in VTI) h is R / 2 and w 1.5 (one pass of two: 0.5); where it holds one, h is 10 and w 0.1.  Past two blocks a CU
+// the blocks partly even out by themselves: x, the mean, has its share beside k.
 // Sweeps of every chunk over ISO FD8, 10, 12, 16 and VTI and TTI FD8, 12, 16 on 18 grids from 40x44x48 to
 // 600x600x400 (MI355X) gave the constants: the rule's chunk takes 1.005 times the best one's time in the mean and
 // 1.08 times at worst (TTI FD8 350x310x370: 0.90 ms, with 11 planes 0.84; ISO at most 1.03).  Asking for 512 blocks
@@ -282,7 +282,10 @@ void Engine::default_tile(int R, bool first_deriv, bool tti, int &etz, int &etx,
   for(int chunk = ny;;) {  // the chunks that cut ny into 1, 2, .. parts, each once
     const double x = tiles * div_up(ny, chunk), k = std::ceil(x);
     const double rounds = std::ceil(0.5 * k);
-    const double cost = (one || k <= 2. ? k + w * rounds : 0.4 * k + 0.6 * x + w * (0.25 * rounds + 0.375 * x)) * (chunk + h);
+    const double waits = k <= 2. ? k + w * rounds
+                         : one   ? 0.5 * (k + x) + w * rounds
+                                 : 0.4 * k + 0.6 * x + w * (0.25 * rounds + 0.375 * x);
+    const double cost = waits * (chunk + h);
     if(eyc <= 0 || cost < best) best = cost, eyc = chunk;
     if(chunk == 1) break;
     chunk = div_up(ny, div_up(ny, chunk - 1));
