@@ -17,7 +17,7 @@
 //  * LDS pitches are constants (an address register and an add per x tap otherwise), blocks that touch no
 //    layer run code without any, and nothing is loaded or stored with the streaming cache policy: a tile's
 //    rows end inside 128-byte lines that its z neighbour reads too (VTI 301x277x333: 20 % less time a step).
-// MI355X, a whole step before and after: TTI FD16 600x600x400 5.45 -> 3.73 ms (14.4 GB moved at 3.8 TB/s, 7.8 GB
+// MI355X, a whole step before and after: TTI FD16 600x600x400 5.46 -> 3.68 ms (14.6 GB moved at 3.9 TB/s, 7.8 GB
 // needed), TTI FD16 300^3 1.19 -> 0.69 ms, VTI FD8 301x277x333 0.96 -> 0.62 ms.
 #pragma once
 #include "fd_tile.h"
